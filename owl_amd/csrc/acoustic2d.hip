@@ -23,6 +23,7 @@
 
 #include "common.hpp"
 #include "host_prep.hpp"
+#include "ordered_sum.hpp"
 #include "owl_amd.h"
 
 namespace owl {
@@ -49,7 +50,7 @@ struct Shot {
     int nr;               // receivers
     int rec0;             // first receiver of the shot in the receiver tables
     int inj0, ninj;       // source injection cells
-    int adj0, nadj;       // adjoint-source injection cells
+    int nadj;             // adjoint-source injection cells
     long long strip0;     // offset of the shot's boundary records
     long long trace0;     // offset of the shot's [nt][nr] trace block
     long long g0;         // offset of the shot's window gradient (nx*nz)
@@ -57,6 +58,7 @@ struct Shot {
     int nxbeg, nzbeg;     // window origin in the full model (1-based)
     int ftile0, fntx;     // fused step: first column-strip tile, strips per row
     int atile0;           // fused adjoint: first column-strip tile (its own z-chunk rows)
+    int rt0, at0;         // sampling and adjoint-source tables (shots of one geometry share them)
     int hnt;              // last reverse step OWL images for this shot (its first source's hnt)
 };
 
@@ -435,16 +437,16 @@ struct Tap {
 // After the update of step t: add_source(t) (module_wavefield.f90:192-263),
 // then sample the receivers for step t+1
 // (submodule_forward_modeling.f90:58-79) and save the boundary record of
-// step t+1 (module_boundary_saving.f90:119-133).  One block per shot, so
-// the samples see the injected source.
+// step t+1 (module_boundary_saving.f90:119-133).  Two launches, because the
+// samples see the injected source: k_inject while a source is active, then
+// k_record over as many blocks as the receivers and strips fill (a single
+// block per shot doing both took 38-42 us per step of the 32-shot batch, as
+// long as one of the sweeps).
 // ---------------------------------------------------------------------------
-template <int R>
-__global__ __launch_bounds__(1024) void k_post_step(
-    const Shot* __restrict__ shots, float* p, float* vx, float* vz,
-    const int* __restrict__ inj_cell_beg, const Tap* __restrict__ inj_taps,
-    const float* __restrict__ amp_tab, int nt, int t, const int* __restrict__ rec_beg,
-    const Tap* __restrict__ rec_taps, const float* __restrict__ rec_w, float* traces, float* strips,
-    int pml) {
+__global__ __launch_bounds__(256) void k_inject(const Shot* __restrict__ shots, float* p, float* vx, float* vz,
+                                                const int* __restrict__ inj_cell_beg,
+                                                const Tap* __restrict__ inj_taps,
+                                                const float* __restrict__ amp_tab, int nt, int t) {
     const Shot S = shots[blockIdx.x];
     // source injection at step t (t in 1..nt); cells in CSR order
     for (int c = threadIdx.x; c < S.ninj; c += blockDim.x) {
@@ -459,32 +461,58 @@ __global__ __launch_bounds__(1024) void k_post_step(
         }
         f[first.cell] = acc;
     }
-    __syncthreads();
-    if (t + 1 > nt) return;
-    for (int r = threadIdx.x; traces && r < S.nr; r += blockDim.x) {
-        const int g = S.rec0 + r;
-        const float w = rec_w[g];
-        float acc = 0.0f;
-        for (int k = rec_beg[g]; k < rec_beg[g + 1]; ++k) {
-            const Tap tp = rec_taps[k];
-            acc = acc + p[tp.cell] * tp.w1 * tp.w2 * w;
-        }
-        traces[S.trace0 + size_t(t) * S.nr + r] = acc;
+}
+
+// One receiver tap, as the sampling reads it: the element within the shot's
+// grid and two weights.  Shots whose receivers lie alike in like windows (a
+// fixed spread) share one table, which then stays in L2: 32 shots of 391
+// off-node receivers read 0.5 MB of taps per step instead of 16 MB.
+struct RecTap {
+    long long cell;
+    float w1, w2;
+};
+// One adjoint-source tap (weights as in the sampling, then the receiver's).
+struct AdjTap {
+    float w1, w2, rw;
+    int row;  // receiver
+};
+
+constexpr int kStripsPerBlock = 1024;  // boundary-record elements a block copies
+
+// Blocks 0 .. nrb-1 of a shot sample `group` receivers each, the others copy
+// its boundary strips (strips != nullptr).
+template <int R>
+__global__ __launch_bounds__(kOrderedThreads) void k_record(
+    const Shot* __restrict__ shots, const float* __restrict__ p, const float* __restrict__ vx,
+    const float* __restrict__ vz, int t, const int* __restrict__ rec_beg, const RecTap* __restrict__ rec_taps,
+    const float* __restrict__ rec_w, float* traces, float* strips, int nrb, int group, int pml) {
+    const Shot S = shots[blockIdx.y];
+    if (int(blockIdx.x) < nrb) {
+        const int r0 = int(blockIdx.x) * group, r1 = min(r0 + group, S.nr);
+        const float* ps = p + S.off;
+        ordered_sums(
+            r0, r1, [&](int r) { return rec_beg[S.rt0 + r]; },
+            [&](int k) {
+                const RecTap tp = rec_taps[k];
+                return ps[tp.cell] * tp.w1 * tp.w2;
+            },
+            [](int) { return 0.0f; }, [&](int r) { return rec_w[S.rec0 + r]; },
+            [&](int r, float acc) { traces[S.trace0 + size_t(t) * S.nr + r] = acc; });
+        return;
     }
-    if (strips) {
-        const int nx = S.nx, nz = S.nz, lo = 1 - pml - R;
-        const int na = R * (nz + 2 * R), nc = (nx + 2 * R) * R;
-        const int len = 2 * na + 2 * nc;
-        float* rec = strips + S.strip0 + size_t(t) * len;
-        for (int k = threadIdx.x; k < len; k += blockDim.x) {
-            int i, j;
-            const float* src;
-            if (k < na) { i = 2 - R + k % R; j = 1 - R + k / R; src = vx; }
-            else if (k < 2 * na) { const int kk = k - na; i = nx + 1 + kk % R; j = 1 - R + kk / R; src = vx; }
-            else if (k < 2 * na + nc) { const int kk = k - 2 * na; i = 1 - R + kk % (nx + 2 * R); j = 2 - R + kk / (nx + 2 * R); src = vz; }
-            else { const int kk = k - 2 * na - nc; i = 1 - R + kk % (nx + 2 * R); j = nz + 1 + kk / (nx + 2 * R); src = vz; }
-            rec[k] = src[size_t(S.off) + size_t(i - lo) + size_t(j - lo) * size_t(S.pitch)];
-        }
+    const int nx = S.nx, nz = S.nz, lo = 1 - pml - R;
+    const int na = R * (nz + 2 * R), nc = (nx + 2 * R) * R;
+    const int len = 2 * na + 2 * nc;
+    float* rec = strips + S.strip0 + size_t(t) * len;
+    const int kb = (int(blockIdx.x) - nrb) * kStripsPerBlock;
+    for (int k = kb + int(threadIdx.x); k < min(kb + kStripsPerBlock, len); k += blockDim.x) {
+        int i, j;
+        const float* src;
+        if (k < na) { i = 2 - R + k % R; j = 1 - R + k / R; src = vx; }
+        else if (k < 2 * na) { const int kk = k - na; i = nx + 1 + kk % R; j = 1 - R + kk / R; src = vx; }
+        else if (k < 2 * na + nc) { const int kk = k - 2 * na; i = 1 - R + kk % (nx + 2 * R); j = 2 - R + kk / (nx + 2 * R); src = vz; }
+        else { const int kk = k - 2 * na - nc; i = 1 - R + kk % (nx + 2 * R); j = nz + 1 + kk / (nx + 2 * R); src = vz; }
+        rec[k] = src[size_t(S.off) + size_t(i - lo) + size_t(j - lo) * size_t(S.pitch)];
     }
 }
 
@@ -525,30 +553,23 @@ __global__ void k_inject_strips(const Shot* __restrict__ shots, float* vx, float
 }
 
 // Adjoint source injection (submodule_fwi_gradient.f90:126-147): cells in CSR
-// order, contributions of each cell in receiver order.
-__device__ __forceinline__ void inject_adjoint_cells(const Shot& S, int c0, int dc, float* pr,
-                                                     const int* __restrict__ cell_beg, const Tap* __restrict__ taps,
-                                                     const float* __restrict__ rec_w, const float* __restrict__ adj,
-                                                     int t) {
-    for (int c = c0; c < S.nadj; c += dc) {
-        const int b = cell_beg[S.adj0 + c], e = cell_beg[S.adj0 + c + 1];
-        const long long cell = taps[b].cell;
-        float acc = pr[cell];
-        for (int k = b; k < e; ++k) {
-            const Tap tp = taps[k];
-            const float a = adj[S.trace0 + size_t(t - 1) * S.nr + tp.row];
-            acc = acc + a * tp.w1 * tp.w2 * rec_w[S.rec0 + tp.row];
-        }
-        pr[cell] = acc;
-    }
-}
-
-__global__ void k_inject_adjoint(const Shot* __restrict__ shots, float* pr,
-                                 const int* __restrict__ cell_beg, const Tap* __restrict__ taps,
-                                 const float* __restrict__ rec_w, const float* __restrict__ adj,
-                                 int t) {
-    inject_adjoint_cells(shots[blockIdx.y], int(blockIdx.x * blockDim.x + threadIdx.x), int(gridDim.x * blockDim.x),
-                         pr, cell_beg, taps, rec_w, adj, t);
+// order, contributions of each cell in receiver order; `group` cells a block.
+__global__ __launch_bounds__(kOrderedThreads) void k_inject_adjoint(
+    const Shot* __restrict__ shots, float* pr, const int* __restrict__ cell_beg,
+    const long long* __restrict__ cells, const AdjTap* __restrict__ taps, const float* __restrict__ adj, int t,
+    int group) {
+    const Shot S = shots[blockIdx.y];
+    const int c0 = int(blockIdx.x) * group, c1 = min(c0 + group, S.nadj);
+    const int* beg = cell_beg + S.at0;
+    const float* a = adj + S.trace0 + size_t(t - 1) * S.nr;
+    ordered_sums(
+        c0, c1, [&](int c) { return beg[c]; },
+        [&](int k) {
+            const AdjTap tp = taps[k];
+            return a[tp.row] * tp.w1 * tp.w2 * tp.rw;
+        },
+        [&](int c) { return pr[S.off + cells[S.at0 + c]]; }, [](int) { return 1.0f; },
+        [&](int c, float acc) { pr[S.off + cells[S.at0 + c]] = acc; });
 }
 
 // Imaging condition of OWL's gradient (submodule_fwi_gradient.f90:201-254,
@@ -1092,10 +1113,11 @@ __global__ __launch_bounds__(256) void k_adj_fused(const Shot* __restrict__ shot
 // The stored p_t includes the source injected at step t; the K gradient
 // needs the increment of the update alone: remove source/K * ph at the
 // source taps active at step t (one block per shot).
-__device__ __forceinline__ void src_correction_cells(const Shot& S, const int* __restrict__ inj_cell_beg,
-                                                     const Tap* __restrict__ inj_taps,
-                                                     const float* __restrict__ amp_tab, const float* __restrict__ bk,
-                                                     const float* ph, double* gK, int nt, int t) {
+__global__ void k_src_correction(const Shot* __restrict__ shots, const int* __restrict__ inj_cell_beg,
+                                 const Tap* __restrict__ inj_taps, const float* __restrict__ amp_tab,
+                                 const float* __restrict__ bk, const float* __restrict__ ph, double* gK,
+                                 int nt, int t) {
+    const Shot S = shots[blockIdx.x];
     for (int c = threadIdx.x; c < S.ninj; c += blockDim.x) {
         const int b = inj_cell_beg[S.inj0 + c], e = inj_cell_beg[S.inj0 + c + 1];
         const long long cell = inj_taps[b].cell;
@@ -1108,31 +1130,6 @@ __device__ __forceinline__ void src_correction_cells(const Shot& S, const int* _
         }
         gK[cell] -= double(src / bk[mq(S, size_t(cell))] * ph[cell]);
     }
-}
-
-__global__ void k_src_correction(const Shot* __restrict__ shots, const int* __restrict__ inj_cell_beg,
-                                 const Tap* __restrict__ inj_taps, const float* __restrict__ amp_tab,
-                                 const float* __restrict__ bk, const float* __restrict__ ph, double* gK,
-                                 int nt, int t) {
-    src_correction_cells(shots[blockIdx.x], inj_cell_beg, inj_taps, amp_tab, bk, ph, gK, nt, t);
-}
-
-// The fused adjoint's tap work of reverse step t in one launch (one block
-// per shot): the source correction (reads ph at the source taps), then the
-// adjoint source injection into ph, in the order of the two kernels above.
-__global__ __launch_bounds__(512) void k_adjoint_taps(const Shot* __restrict__ shots,
-                                                      const int* __restrict__ inj_cell_beg,
-                                                      const Tap* __restrict__ inj_taps,
-                                                      const float* __restrict__ amp_tab,
-                                                      const float* __restrict__ bk, float* ph, double* gK, int nt,
-                                                      const int* __restrict__ adj_beg,
-                                                      const Tap* __restrict__ adj_taps,
-                                                      const float* __restrict__ rec_w, const float* __restrict__ adj,
-                                                      int t) {
-    const Shot S = shots[blockIdx.x];
-    src_correction_cells(S, inj_cell_beg, inj_taps, amp_tab, bk, ph, gK, nt, t);
-    __syncthreads();
-    inject_adjoint_cells(S, int(threadIdx.x), int(blockDim.x), ph, adj_beg, adj_taps, rec_w, adj, t);
 }
 
 // Fold the padded-grid gradients onto the window (edge replication
@@ -1389,7 +1386,12 @@ struct owl_acoustic2d {
     DevBuf<float> aF[3], aM[4];         // adjoint field and PML memory
     DevBuf<float> d_amp;                // source amplitude rows [row][nt]
     DevBuf<int> d_inj_beg, d_adj_beg, d_rec_beg;
-    DevBuf<Tap> d_inj_taps, d_adj_taps, d_rec_taps;
+    DevBuf<Tap> d_inj_taps;
+    DevBuf<AdjTap> d_adj_taps;
+    DevBuf<long long> d_adj_cell;       // element of each adjoint-source cell within its shot's grid
+    DevBuf<RecTap> d_rec_taps;
+    int rec_group = 1, adj_group = 1;   // sums per block of the sampling and the adjoint injection
+    int max_nr = 0, max_strip = 0;      // largest receiver count and boundary record of one shot
     DevBuf<float> d_rec_w;
     DevBuf<float> d_traces, d_obs, d_adj, d_strips, d_edge;
     DevBuf<double> d_gv, d_gr, d_gfull_v, d_gfull_r, d_misfit, d_scratch;
@@ -1568,14 +1570,19 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     long long off = 0, moff = 0, strip = 0, trace = 0, g0 = 0;
     int edge = 0, prof = 0;
     std::vector<float> profs, amp;
-    std::vector<int> inj_beg{0}, adj_beg{0}, rec_beg{0};
-    std::vector<Tap> inj_taps, adj_taps, rec_taps;
+    std::vector<int> inj_beg{0}, adj_beg, rec_beg;
+    std::vector<Tap> inj_taps;
+    std::vector<AdjTap> adj_taps;
+    std::vector<long long> adj_cell;
+    std::vector<RecTap> rec_taps;
     std::vector<float> rec_w;
     b->pts_full = 0;
     b->pts_model = 0;
     b->nrec_total = 0;   // every per-plan table is rebuilt from zero
     b->max_ninj = 0;
     b->max_nadj = 0;
+    b->max_nr = 0;
+    b->max_strip = 0;
     b->src_t0 = 1 << 30;
     b->src_t1 = -1;
     for (int s = 0; s < nshot; ++s) {
@@ -1741,39 +1748,78 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
         if (!st.empty()) inj_beg.push_back(int(inj_taps.size()));
         b->max_ninj = std::max(b->max_ninj, S.ninj);
 
-        // ---- receivers (prepare_geometry; sampling and adjoint injection)
+        // ---- receivers (prepare_geometry; sampling and adjoint injection):
+        // tables relative to the shot's grid, shared with an earlier shot of
+        // the same grid whose receivers give the same ones
         S.rec0 = b->nrec_total;
-        std::vector<Tap> at;
+        std::vector<RecTap> rt;
+        std::vector<int> rb{0};
+        std::vector<float> rw;
         for (int r = 0; r < S.nr; ++r) {
             const owl_receiver& rc = H.rec[r];
             const bool valid = rc.x >= H.ox && rc.x <= xmax && rc.z >= H.oz && rc.z <= zmax;
             const float w = (valid && rc.weight != 0.f) ? rc.weight : 0.f;
-            rec_w.push_back(w);
+            rw.push_back(w);
             if (w != 0.f) {
                 const Located L = locate(2, rc.x, 0.f, rc.z, H.ox, 0.f, H.oz, cfg->dx, 1.f, cfg->dz);
                 for (int irz = -kNkw; irz <= kNkw; ++irz)
                     for (int irx = -kNkw; irx <= kNkw; ++irx) {
                         const float w1 = L.ix[irx + kNkw], w2 = L.iz[irz + kNkw];
                         if (w1 == 0.f || w2 == 0.f) continue;
-                        const Tap tp{(long long)cell_of(b, S, L.gx + irx, L.gz + irz), w1, w2, r, 0, 0, 0};
-                        rec_taps.push_back(tp);
-                        at.push_back(tp);
+                        rt.push_back(RecTap{(long long)cell_of(b, S, L.gx + irx, L.gz + irz) - S.off, w1, w2});
                     }
             }
-            rec_beg.push_back(int(rec_taps.size()));
+            rb.push_back(int(rt.size()));
+        }
+        int same = -1;
+        for (int u = 0; u < s && same < 0; ++u) {
+            const Shot& U = b->sd[u];
+            if (U.nr != S.nr || U.pitch != S.pitch || U.nrow != S.nrow || (u > 0 && U.rt0 == b->sd[u - 1].rt0)) continue;
+            const int k0 = rec_beg[size_t(U.rt0)];
+            bool eq = std::equal(rw.begin(), rw.end(), rec_w.begin() + U.rec0);
+            for (int r = 0; r <= S.nr && eq; ++r) eq = rec_beg[size_t(U.rt0 + r)] - k0 == rb[size_t(r)];
+            for (size_t k = 0; k < rt.size() && eq; ++k) {
+                const RecTap& q = rec_taps[size_t(k0) + k];
+                eq = q.cell == rt[k].cell && q.w1 == rt[k].w1 && q.w2 == rt[k].w2;
+            }
+            if (eq) same = u;
+        }
+        rec_w.insert(rec_w.end(), rw.begin(), rw.end());
+        if (same >= 0) {
+            S.rt0 = b->sd[same].rt0;
+            S.at0 = b->sd[same].at0;
+            S.nadj = b->sd[same].nadj;
+        } else {
+            S.rt0 = int(rec_beg.size());
+            const int k0 = int(rec_taps.size());
+            for (int k : rb) rec_beg.push_back(k0 + k);
+            rec_taps.insert(rec_taps.end(), rt.begin(), rt.end());
+            // adjoint source: the same taps by cell, in receiver order
+            struct Hit {
+                long long cell;
+                AdjTap tap;
+            };
+            std::vector<Hit> at;
+            for (int r = 0; r < S.nr; ++r)
+                for (int k = rb[size_t(r)]; k < rb[size_t(r) + 1]; ++k)
+                    at.push_back(Hit{rt[size_t(k)].cell, AdjTap{rt[size_t(k)].w1, rt[size_t(k)].w2, rw[size_t(r)], r}});
+            std::stable_sort(at.begin(), at.end(), [](const Hit& x, const Hit& y) { return x.cell < y.cell; });
+            S.at0 = int(adj_beg.size());
+            S.nadj = 0;
+            for (size_t k = 0; k < at.size(); ++k) {
+                if (k == 0 || at[k].cell != at[k - 1].cell) {
+                    adj_beg.push_back(int(adj_taps.size()));
+                    adj_cell.push_back(at[k].cell);
+                    ++S.nadj;
+                }
+                adj_taps.push_back(at[k].tap);
+            }
+            adj_beg.push_back(int(adj_taps.size()));  // end of the last cell; keeps beg and cell aligned
+            adj_cell.push_back(0);
         }
         b->nrec_total += S.nr;
-        std::stable_sort(at.begin(), at.end(), [](const Tap& a, const Tap& c) { return a.cell < c.cell; });
-        S.adj0 = int(adj_beg.size()) - 1;
-        S.nadj = 0;
-        for (size_t k = 0; k < at.size(); ++k) {
-            if (k == 0 || at[k].cell != at[k - 1].cell) {
-                if (k) adj_beg.push_back(int(adj_taps.size()));
-                ++S.nadj;
-            }
-            adj_taps.push_back(at[k]);
-        }
-        if (!at.empty()) adj_beg.push_back(int(adj_taps.size()));
+        b->max_nr = std::max(b->max_nr, S.nr);
+        b->max_strip = std::max(b->max_strip, strip_len);
         b->max_nadj = std::max(b->max_nadj, S.nadj);
     }
     b->field_elems = size_t(off);
@@ -1789,9 +1835,9 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
         const Shot& S = b->sd[s];
         const bool ok =
             S.rec0 >= 0 && size_t(S.rec0) + size_t(S.nr) <= rec_w.size() &&
-            size_t(S.rec0) + size_t(S.nr) + 1 <= rec_beg.size() &&
+            S.rt0 >= 0 && size_t(S.rt0) + size_t(S.nr) + 1 <= rec_beg.size() &&
             S.inj0 >= 0 && size_t(S.inj0) + size_t(S.ninj) + (S.ninj ? 1 : 0) <= inj_beg.size() &&
-            S.adj0 >= 0 && size_t(S.adj0) + size_t(S.nadj) + (S.nadj ? 1 : 0) <= adj_beg.size() &&
+            S.at0 >= 0 && size_t(S.at0) + size_t(S.nadj) + 1 <= adj_beg.size() && adj_cell.size() == adj_beg.size() &&
             size_t(S.trace0) + size_t(nt) * size_t(S.nr) <= b->trace_elems &&
             size_t(S.strip0) + size_t(nt) * size_t(2 * R * (S.nz + 2 * R) + 2 * (S.nx + 2 * R) * R) <= b->strip_elems &&
             size_t(S.g0) + size_t(S.nx) * size_t(S.nz) <= b->grad_elems &&
@@ -1804,7 +1850,7 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     for (const Tap& tp : inj_taps)
         if (tp.cell < 0 || size_t(tp.cell) >= b->field_elems || size_t(tp.row + 1) * nt > amp.size())
             fail(OWL_ERR_ARG, "internal layout check failed for a source tap");
-    for (const Tap& tp : rec_taps)
+    for (const RecTap& tp : rec_taps)  // cell_of has checked each against its shot's grid
         if (tp.cell < 0 || size_t(tp.cell) >= b->field_elems) fail(OWL_ERR_ARG, "internal layout check failed for a receiver tap");
 
     if (!b->stream) {
@@ -1826,10 +1872,13 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     if (inj_taps.empty()) inj_taps.push_back(Tap{});
     b->d_inj_taps.upload(inj_taps, st);
     b->d_rec_beg.upload(rec_beg, st);
-    if (rec_taps.empty()) rec_taps.push_back(Tap{});
+    b->rec_group = ordered_group(rec_beg);
+    b->adj_group = ordered_group(adj_beg);
+    if (rec_taps.empty()) rec_taps.push_back(RecTap{});
     b->d_rec_taps.upload(rec_taps, st);
     b->d_adj_beg.upload(adj_beg, st);
-    if (adj_taps.empty()) adj_taps.push_back(Tap{});
+    if (adj_taps.empty()) adj_taps.push_back(AdjTap{});
+    b->d_adj_cell.upload(adj_cell, st);
     b->d_adj_taps.upload(adj_taps, st);
     b->d_rec_w.upload(rec_w, st);
     for (int k = 0; k < 3; ++k) b->fA[k].alloc(b->field_elems);
@@ -1942,6 +1991,38 @@ void launch_step(owl_acoustic2d* b, const Sets& sets, int nsets, float dt) {
     prof_end(b, ev);
 }
 
+// The source of step t and, unless null, the receivers (and boundary record)
+// of step t+1.  Outside every source's active steps the injection would
+// change nothing and is not launched.
+template <int R>
+void post_step(owl_acoustic2d* b, float* const* f, int t, float* traces, float* strips) {
+    const unsigned nshot = unsigned(b->sd.size());
+    if (t >= b->src_t0 && t <= b->src_t1) {
+        const int ev = prof_begin(b, kKPost);
+        hipLaunchKernelGGL(k_inject, dim3(nshot), dim3(256), 0, b->stream, b->d_shots.get(), f[0], f[1], f[2],
+                           b->d_inj_beg.get(), b->d_inj_taps.get(), b->d_amp.get(), b->nt, t);
+        prof_end(b, ev);
+    }
+    if (!traces || t + 1 > b->nt) return;
+    const int nrb = (b->max_nr + b->rec_group - 1) / b->rec_group;
+    const int nsb = strips ? (b->max_strip + kStripsPerBlock - 1) / kStripsPerBlock : 0;
+    const int ev = prof_begin(b, kKPost);
+    hipLaunchKernelGGL(k_record<R>, dim3(unsigned(nrb + nsb), nshot), dim3(kOrderedThreads), 0, b->stream,
+                       b->d_shots.get(), f[0], f[1], f[2], t, b->d_rec_beg.get(), b->d_rec_taps.get(),
+                       b->d_rec_w.get(), traces, strips, nrb, b->rec_group, b->pml);
+    prof_end(b, ev);
+}
+
+void launch_inject_adjoint(owl_acoustic2d* b, float* pr, int t) {
+    if (b->max_nadj <= 0) return;
+    const int ev = prof_begin(b, kKAdj);
+    hipLaunchKernelGGL(k_inject_adjoint, dim3(unsigned((b->max_nadj + b->adj_group - 1) / b->adj_group),
+                                              unsigned(b->sd.size())),
+                       dim3(kOrderedThreads), 0, b->stream, b->d_shots.get(), pr, b->d_adj_beg.get(),
+                       b->d_adj_cell.get(), b->d_adj_taps.get(), b->d_adj.get(), t, b->adj_group);
+    prof_end(b, ev);
+}
+
 template <int R>
 void run_forward(owl_acoustic2d* b, bool save) {
     hipStream_t st = b->stream;
@@ -1956,20 +2037,14 @@ void run_forward(owl_acoustic2d* b, bool save) {
     }
     float* m[4] = {b->fM[0].get(), b->fM[1].get(), b->fM[2].get(), b->fM[3].get()};
     const Sets sets = one_set(b->fA[0].get(), b->fA[1].get(), b->fA[2].get(), m);
-    const unsigned nshot = unsigned(b->sd.size());
     OWL_HIP(hipEventRecord(b->ev0, st));
     // steps 1..nt-1; the update and source of step nt change nothing that
     // OWL records, and skipping them leaves the state of the start of step nt
     // (OWL's output_final_step_wavefield) in place.
     for (int t = 1; t <= b->nt - 1; ++t) {
         launch_step<R>(b, sets, 1, b->dt);
-        const int ev = prof_begin(b, kKPost);
-        hipLaunchKernelGGL(k_post_step<R>, dim3(nshot), dim3(512), 0, st, b->d_shots.get(),
-                           b->fA[0].get(), b->fA[1].get(), b->fA[2].get(), b->d_inj_beg.get(),
-                           b->d_inj_taps.get(), b->d_amp.get(), b->nt, t, b->d_rec_beg.get(),
-                           b->d_rec_taps.get(), b->d_rec_w.get(), b->d_traces.get(),
-                           save ? b->d_strips.get() : nullptr, b->pml);
-        prof_end(b, ev);
+        float* f[3] = {b->fA[0].get(), b->fA[1].get(), b->fA[2].get()};
+        post_step<R>(b, f, t, b->d_traces.get(), save ? b->d_strips.get() : nullptr);
     }
     OWL_HIP(hipGetLastError());
     OWL_HIP(hipEventRecord(b->ev1, st));
@@ -2040,12 +2115,7 @@ void run_reverse_owl(owl_acoustic2d* b) {
         sets.s[0].vz_out = B[2].get();
         sets.s[1] = in_place(b->aF[0].get(), b->aF[1].get(), b->aF[2].get(), am);
         launch_step<R>(b, sets, 2, -b->dt);
-        ev = prof_begin(b, kKAdj);
-        if (b->max_nadj > 0)
-            hipLaunchKernelGGL(k_inject_adjoint, dim3(unsigned((b->max_nadj + 255) / 256), nshot), dim3(256), 0,
-                               st, b->d_shots.get(), b->aF[0].get(), b->d_adj_beg.get(),
-                               b->d_adj_taps.get(), b->d_rec_w.get(), b->d_adj.get(), t);
-        prof_end(b, ev);
+        launch_inject_adjoint(b, b->aF[0].get(), t);
         ev = prof_begin(b, kKImage, (t % cc == 0) ? image_bytes : 0.0);
         if (t % cc == 0)
             hipLaunchKernelGGL(k_image_owl<R>, dim3(ig, nshot), dim3(256), 0, st, b->d_shots.get(),
@@ -2163,15 +2233,7 @@ void fwd_step(owl_acoustic2d* b, const W7& in, const W7& out, int t, bool record
     } else {
         launch_step<R>(b, sets, 1, b->dt);
     }
-    // without receivers to sample and outside every source's active steps the
-    // post-step kernel would change nothing
-    if (!record && (t < b->src_t0 || t > b->src_t1)) return;
-    const int ev = prof_begin(b, kKPost);
-    hipLaunchKernelGGL(k_post_step<R>, dim3(unsigned(b->sd.size())), dim3(512), 0, b->stream, b->d_shots.get(),
-                       out.f[0], out.f[1], out.f[2], b->d_inj_beg.get(), b->d_inj_taps.get(), b->d_amp.get(),
-                       b->nt, t, b->d_rec_beg.get(), b->d_rec_taps.get(), b->d_rec_w.get(),
-                       record ? b->d_traces.get() : nullptr, nullptr, b->pml);
-    prof_end(b, ev);
+    post_step<R>(b, out.f, t, record ? b->d_traces.get() : nullptr, nullptr);
 }
 
 // Clear device memory on the batch stream: a memset, or a fill kernel while
@@ -2293,13 +2355,16 @@ void adjoint_alloc_zero(owl_acoustic2d* b) {
 // between adj[0] and adj2[0]).
 float* cur_ph(owl_acoustic2d* b) { return b->adj_cur ? b->adj2[0].get() : b->adj[0].get(); }
 
-void inject_residual(owl_acoustic2d* b, int t) {
-    const unsigned nshot = unsigned(b->sd.size());
-    if (b->max_nadj <= 0) return;
+void inject_residual(owl_acoustic2d* b, int t) { launch_inject_adjoint(b, cur_ph(b), t); }
+
+// Remove the source of step t from the K gradient (nothing to remove
+// outside every source's active steps).
+void src_correction(owl_acoustic2d* b, int t) {
+    if (b->max_ninj <= 0 || t < b->src_t0 || t > b->src_t1) return;
     const int ev = prof_begin(b, kKAdj);
-    hipLaunchKernelGGL(k_inject_adjoint, dim3(unsigned((b->max_nadj + 255) / 256), nshot), dim3(256), 0, b->stream,
-                       b->d_shots.get(), cur_ph(b), b->d_adj_beg.get(), b->d_adj_taps.get(),
-                       b->d_rec_w.get(), b->d_adj.get(), t);
+    hipLaunchKernelGGL(k_src_correction, dim3(unsigned(b->sd.size())), dim3(256), 0, b->stream, b->d_shots.get(),
+                       b->d_inj_beg.get(), b->d_inj_taps.get(), b->d_amp.get(), b->d_bk.get(), cur_ph(b),
+                       b->gK.get(), b->nt, t);
     prof_end(b, ev);
 }
 
@@ -2330,14 +2395,8 @@ void adjoint_step(owl_acoustic2d* b, int t, const float* const* cur, const float
                            prev[1], cur[2], prev[2]);
         prof_end(b, ev);
         b->adj_cur = 1 - b->adj_cur;
-        if (b->max_ninj > 0 || b->max_nadj > 0) {
-            const int ev2 = prof_begin(b, kKAdj);
-            hipLaunchKernelGGL(k_adjoint_taps, dim3(unsigned(b->sd.size())), dim3(512), 0, b->stream,
-                               b->d_shots.get(), b->d_inj_beg.get(), b->d_inj_taps.get(), b->d_amp.get(),
-                               b->d_bk.get(), cur_ph(b), b->gK.get(), b->nt, b->d_adj_beg.get(),
-                               b->d_adj_taps.get(), b->d_rec_w.get(), b->d_adj.get(), t);
-            prof_end(b, ev2);
-        }
+        src_correction(b, t);
+        inject_residual(b, t);
         return;
     }
     // p-pass: ex, ez, ph, bk, p_t, p_{t-1}, psx/psz read; ph, dx, dz written; gK r+w
@@ -2345,10 +2404,7 @@ void adjoint_step(owl_acoustic2d* b, int t, const float* const* cur, const float
     hipLaunchKernelGGL(k_adj_p<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), A, b->d_bk.get(),
                        b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, cur[0], prev[0]);
     prof_end(b, ev);
-    if (b->max_ninj > 0)
-        hipLaunchKernelGGL(k_src_correction, dim3(unsigned(b->sd.size())), dim3(256), 0, b->stream, b->d_shots.get(),
-                           b->d_inj_beg.get(), b->d_inj_taps.get(), b->d_amp.get(), b->d_bk.get(), b->adj[0].get(),
-                           b->gK.get(), b->nt, t);
+    src_correction(b, t);
     // v-pass: dx, dz, vxh, vzh, rho, 4 states read; vxh, vzh, ex, ez written; gX, gZ r+w
     ev = prof_begin(b, 11, pts * (8 * 4 + 4 * 4 + 32) + 4.0 * b->pts_model);
     hipLaunchKernelGGL(k_adj_v<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), A, b->d_rho.get(),
@@ -2857,7 +2913,7 @@ std::vector<uintptr_t> exact_signature(owl_acoustic2d* b, int ckpt, int param, i
         add(f->get());
     add(b->d_shots.get()); add(b->d_tile_shot.get()); add(b->d_ftile_shot.get()); add(b->d_atile_shot.get());
     add(b->d_inj_beg.get()); add(b->d_adj_beg.get()); add(b->d_rec_beg.get());
-    add(b->d_inj_taps.get()); add(b->d_adj_taps.get()); add(b->d_rec_taps.get());
+    add(b->d_inj_taps.get()); add(b->d_adj_taps.get()); add(b->d_adj_cell.get()); add(b->d_rec_taps.get());
     return v;
 }
 

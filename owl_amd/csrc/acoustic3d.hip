@@ -20,6 +20,7 @@
 
 #include "common.hpp"
 #include "host_prep.hpp"
+#include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
 
@@ -1232,19 +1233,17 @@ __global__ __launch_bounds__(64 * kFW) void k3f_step(const Shot3* __restrict__ s
 }
 
 // Source injection of step t (add_source, module_wavefield.f90:322-444:
-// explosions into p, forces into vx, vy, vz) then receivers of step t+1;
-// one block per shot so that the samples see the injected source.  Taps are
-// grouped by (field, cell); the contributions to one cell are added in
-// source order.
-__global__ __launch_bounds__(1024) void k3_post_step(const Shot3* __restrict__ shots, float* p, float* vx,
-                                                     float* vy, float* vz, const int* __restrict__ inj_beg,
-                                                     const Tap3* __restrict__ inj,
-                                                     const float* __restrict__ amp_tab, int nt, int t,
-                                                     const int* __restrict__ rec_beg,
-                                                     const Tap3* __restrict__ rec,
-                                                     const float* __restrict__ rec_w, float* traces) {
-    const Shot3 S = shots[blockIdx.x];
-    for (int c = threadIdx.x; c < S.ninj; c += blockDim.x) {
+// explosions into p, forces into vx, vy, vz), launched while a source is
+// active; the receivers of step t+1 follow in a launch of their own
+// (k3_record), so that the samples see the injected source and spread over
+// the chip.  Taps are grouped by (field, cell); the contributions to one
+// cell are added in source order.
+__global__ __launch_bounds__(256) void k3_inject(const Shot3* __restrict__ shots, float* p, float* vx, float* vy,
+                                                 float* vz, const int* __restrict__ inj_beg,
+                                                 const Tap3* __restrict__ inj, const float* __restrict__ amp_tab,
+                                                 int nt, int t) {
+    const Shot3 S = shots[blockIdx.y];
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < S.ninj; c += gridDim.x * blockDim.x) {
         const int b = inj_beg[S.inj0 + c], e = inj_beg[S.inj0 + c + 1];
         const long long cell = inj[b].cell;
         const int fld = inj[b].field;
@@ -1257,18 +1256,31 @@ __global__ __launch_bounds__(1024) void k3_post_step(const Shot3* __restrict__ s
         }
         f[cell] = acc;
     }
-    __syncthreads();
-    if (t + 1 > nt || !traces) return;
-    for (int r = threadIdx.x; r < S.nr; r += blockDim.x) {
-        const int g = S.rec0 + r;
-        const float w = rec_w[g];
-        float acc = 0.0f;
-        for (int k = rec_beg[g]; k < rec_beg[g + 1]; ++k) {
-            const Tap3 tp = rec[k];
-            acc = acc + p[tp.cell] * tp.w1 * tp.w2 * tp.w3 * w;
-        }
-        traces[S.trace0 + size_t(t) * S.nr + r] = acc;
-    }
+}
+
+// One receiver tap, as the sampling reads it.
+struct RecTap3 {
+    long long cell;
+    float w1, w2, w3;
+};
+
+// Receivers of step t+1, `group` to a block.
+__global__ __launch_bounds__(kOrderedThreads) void k3_record(const Shot3* __restrict__ shots,
+                                                             const float* __restrict__ p, int t,
+                                                             const int* __restrict__ rec_beg,
+                                                             const RecTap3* __restrict__ rec,
+                                                             const float* __restrict__ rec_w, float* traces,
+                                                             int group) {
+    const Shot3 S = shots[blockIdx.y];
+    const int r0 = int(blockIdx.x) * group, r1 = min(r0 + group, S.nr);
+    ordered_sums(
+        r0, r1, [&](int r) { return rec_beg[S.rec0 + r]; },
+        [&](int k) {
+            const RecTap3 tp = rec[k];
+            return p[tp.cell] * tp.w1 * tp.w2 * tp.w3;
+        },
+        [](int) { return 0.0f; }, [&](int r) { return rec_w[S.rec0 + r]; },
+        [&](int r, float acc) { traces[S.trace0 + size_t(t) * S.nr + r] = acc; });
 }
 
 // Free surface: p(:,:,k) = -p(:,:,2-k) for k <= 0 (module_wavefield.f90:240-250).
@@ -1569,7 +1581,11 @@ struct owl_acoustic3d {
     DevBuf<float> aF[4], aM[6];          // adjoint state
     DevBuf<float> d_strips, d_edge;
     DevBuf<double> d_gv, d_gr, d_gfull_v, d_gfull_r, d_misfit, d_scratch;
-    DevBuf<Tap3> d_inj, d_rec, d_adj_taps;
+    DevBuf<Tap3> d_inj, d_adj_taps;
+    DevBuf<RecTap3> d_rec;
+    int rec_group = 1;                 // receivers per block of the sampling
+    int max_nr = 0;
+    int src_t0 = 1, src_t1 = 0;        // steps during which any source tap is active
     bool have_boundary = false, fwd_state_valid = false, have_obs = false;
     // HIP graph of the forward time loop (modelling without boundary
     // records, profiling off): captured by the first such call, replayed by
@@ -1702,14 +1718,17 @@ void plan3(owl_acoustic3d* b, const owl_acoustic_config* cfg, const float* vp, c
     b->sd.assign(nshot, Shot3{});
     b->tile_shot.clear();
     b->nrec_total = 0;
-    b->max_ninj = b->max_nadj = 0;
+    b->max_ninj = b->max_nadj = b->max_nr = 0;
+    b->src_t0 = 1 << 30;
+    b->src_t1 = -1;
     b->pts_full = 0;
     b->have_boundary = b->fwd_state_valid = b->have_obs = false;
     long long off = 0, trace = 0, strip = 0, edge = 0, grad = 0;
     int prof = 0;
     std::vector<float> profs, amp, rec_w;
     std::vector<int> inj_beg{0}, rec_beg{0}, adj_beg{0};
-    std::vector<Tap3> inj, rec, adjt;
+    std::vector<Tap3> inj, adjt;
+    std::vector<RecTap3> rec;
     for (int s = 0; s < nshot; ++s) {
         const owl_shot& in = shots[s];
         ShotHost3& H = b->hs[s];
@@ -1805,6 +1824,8 @@ void plan3(owl_acoustic3d* b, const owl_acoustic_config* cfg, const float* vp, c
                 S.hnt = std::max(hnt, 1);
             }
             const int nbeg = fortran_nint(sc.t0 / cfg->dt) + 1, nend = nbeg + int(stf.size()) - 1;
+            b->src_t0 = std::min(b->src_t0, nbeg);
+            b->src_t1 = std::max(b->src_t1, nend);
             std::vector<float> a(nt, 0.f);
             for (int t = std::max(nbeg, 1); t <= std::min(nend, nt); ++t) a[t - 1] = stf[t - nbeg] * sc.amp * cfg->dt;
             auto add_taps = [&](int field, int gx, int gy, int gz, const float* wx, const float* wy, const float* wz,
@@ -1861,7 +1882,7 @@ void plan3(owl_acoustic3d* b, const owl_acoustic_config* cfg, const float* vp, c
                             if (w1 == 0.f || w2 == 0.f || w3 == 0.f) continue;
                             const Tap3 tp{(long long)cell3(b, S, L.gx + irx, L.gy + iry, L.gz + irz), w1, w2, w3, r,
                                           0, 0, 0};
-                            rec.push_back(tp);
+                            rec.push_back(RecTap3{tp.cell, w1, w2, w3});
                             at.push_back(tp);
                         }
             }
@@ -1871,6 +1892,7 @@ void plan3(owl_acoustic3d* b, const owl_acoustic_config* cfg, const float* vp, c
         S.adj0 = int(adj_beg.size()) - 1;
         S.nadj = csr_by_cell(at, adj_beg, adjt);
         b->max_nadj = std::max(b->max_nadj, S.nadj);
+        b->max_nr = std::max(b->max_nr, S.nr);
         b->nrec_total += S.nr;
     }
     b->field_elems = size_t(off);
@@ -1900,7 +1922,8 @@ void plan3(owl_acoustic3d* b, const owl_acoustic_config* cfg, const float* vp, c
     if (inj.empty()) inj.push_back(Tap3{});
     b->d_inj.upload(inj, stm);
     b->d_rec_beg.upload(rec_beg, stm);
-    if (rec.empty()) rec.push_back(Tap3{});
+    b->rec_group = ordered_group(rec_beg);
+    if (rec.empty()) rec.push_back(RecTap3{});
     b->d_rec.upload(rec, stm);
     b->d_rec_w.upload(rec_w, stm);
     b->d_adj_beg.upload(adj_beg, stm);
@@ -2129,11 +2152,19 @@ void run_forward3(owl_acoustic3d* b, bool save_boundary) {
             } else {
                 sweeps3<R>(b, F, b->dt);
             }
+            // outside every source's active steps the injection would change nothing
+            if (b->max_ninj > 0 && t >= b->src_t0 && t <= b->src_t1) {
+                const int ev = b->prof.begin(st, 2, 0);
+                hipLaunchKernelGGL(k3_inject, dim3(unsigned((b->max_ninj + 255) / 256), unsigned(b->sd.size())),
+                                   dim3(256), 0, st, b->d_shots.get(), cur.f[0], cur.f[1], cur.f[2], cur.f[3],
+                                   b->d_inj_beg.get(), b->d_inj.get(), b->d_amp.get(), b->nt, t);
+                b->prof.end(st, ev);
+            }
             const int ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(k3_post_step, dim3(unsigned(b->sd.size())), dim3(1024), 0, st, b->d_shots.get(),
-                               cur.f[0], cur.f[1], cur.f[2], cur.f[3], b->d_inj_beg.get(),
-                               b->d_inj.get(), b->d_amp.get(), b->nt, t, b->d_rec_beg.get(), b->d_rec.get(),
-                               b->d_rec_w.get(), b->d_traces.get());
+            hipLaunchKernelGGL(k3_record, dim3(unsigned((b->max_nr + b->rec_group - 1) / b->rec_group),
+                                               unsigned(b->sd.size())),
+                               dim3(kOrderedThreads), 0, st, b->d_shots.get(), cur.f[0], t, b->d_rec_beg.get(),
+                               b->d_rec.get(), b->d_rec_w.get(), b->d_traces.get(), b->rec_group);
             b->prof.end(st, ev);
             if (!b->graph.capturing) maybe_collect(b);
         }

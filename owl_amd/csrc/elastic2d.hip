@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "fs_mesh.hpp"
 #include "host_prep.hpp"
+#include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
 #include "record_store.hpp"
@@ -345,24 +346,27 @@ __global__ __launch_bounds__(1024) void k2e_inject(const ShotE2* __restrict__ sh
     }
 }
 
-// Receivers of step t: vx at (hx, gz), vz at (gx, hz).
-__global__ __launch_bounds__(256) void k2e_record(const ShotE2* __restrict__ shots, const float* __restrict__ vx,
-                                                  const float* __restrict__ vz, const int* __restrict__ rec_beg,
-                                                  const Tap* __restrict__ rec, const float* __restrict__ rec_w,
-                                                  float* traces, int nt, int t) {
+// Receivers of step t: vx at (hx, gz), vz at (gx, hz); `group` components
+// of a shot's 2 nr to a block.
+__global__ __launch_bounds__(kOrderedThreads) void k2e_record(
+    const ShotE2* __restrict__ shots, const float* __restrict__ vx, const float* __restrict__ vz,
+    const int* __restrict__ rec_beg, const Tap* __restrict__ rec, const float* __restrict__ rec_w, float* traces,
+    int nt, int t, int group) {
     const ShotE2 S = shots[blockIdx.y];
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < 2 * S.nr; r += gridDim.x * blockDim.x) {
-        const int comp = r / S.nr, ir = r % S.nr;
-        const int g = 2 * S.rec0 + comp * S.nr + ir;
-        const float w = rec_w[S.rec0 + ir];
-        const float* f = comp == 0 ? vx : vz;
-        float acc = 0.0f;
-        for (int k = rec_beg[g]; k < rec_beg[g + 1]; ++k) {
+    const int r0 = int(blockIdx.x) * group, r1 = min(r0 + group, 2 * S.nr);
+    const int* beg = rec_beg + 2 * S.rec0;
+    ordered_sums(
+        r0, r1, [&](int r) { return beg[r]; },
+        [&](int k) {
             const Tap tp = rec[k];
-            acc = acc + f[tp.cell] * tp.w1 * tp.w2 * w;
-        }
-        traces[S.trace0 + size_t(comp) * nt * S.nr + size_t(t - 1) * S.nr + ir] = acc;
-    }
+            return (k < beg[S.nr] ? vx : vz)[tp.cell] * tp.w1 * tp.w2;
+        },
+        [](int) { return 0.0f; },
+        [&](int r) { return rec_w[S.rec0 + (r < S.nr ? r : r - S.nr)]; },
+        [&](int r, float acc) {
+            const int comp = r < S.nr ? 0 : 1, ir = r - comp * S.nr;
+            traces[S.trace0 + size_t(comp) * nt * S.nr + size_t(t - 1) * S.nr + ir] = acc;
+        });
 }
 
 // Boundary records (module_boundary_saving.f90:89-160): for vx, then vz:
@@ -557,6 +561,8 @@ struct owl_elastic2d {
     DevBuf<float> fB[5];    // the other half of the reverse ping-pong
     DevBuf<float> aF[13];   // adjoint field
     DevBuf<Tap> d_inj, d_rec, d_adj_taps;
+    int rec_group = 1;                 // receivers per block of the sampling
+    int src_t0 = 1, src_t1 = 0;        // steps during which any source tap is active
     DevBuf<double> d_gA, d_gB, d_gC, d_fA, d_fB, d_fC, d_misfit, d_scratch;
     // the forward time loop as one HIP graph (modelling without profiling
     // or boundary records), re-captured when a launch argument changes
@@ -684,6 +690,8 @@ void plan2(owl_elastic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     b->hs.assign(nshot, ShotHostE2{});
     b->sd.assign(nshot, ShotE2{});
     b->nrec_total = b->max_nr = b->max_nadj = 0;
+    b->src_t0 = 1 << 30;
+    b->src_t1 = -1;
     b->pts_full = 0;
     b->mesh.assign(b->fs ? size_t(nshot) : 0, fsm::SsgMesh{});
     b->rho_map.assign(b->fs ? size_t(nshot) : 0, std::vector<float>{});
@@ -853,6 +861,8 @@ void plan2(owl_elastic2d* b, const owl_acoustic_config* cfg, const float* vp, co
                 S.hnt = std::max(hnt, 1);
             }
             const int nbeg = fortran_nint(sc.t0 / cfg->dt) + 1, nend = nbeg + int(stf.size()) - 1;
+            b->src_t0 = std::min(b->src_t0, nbeg);
+            b->src_t1 = std::max(b->src_t1, nend);
             if (sc.mechanism == OWL_EXPLOSION) {
                 // the stress drop divides by the local spacing dz_i(gz) on the refined mesh
                 const float dzs = Ms ? Ms->dzi[size_t(L.gz + pml)] : cfg->dz;
@@ -993,6 +1003,7 @@ void plan2(owl_elastic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     if (inj.empty()) inj.push_back(Tap{});
     b->d_inj.upload(inj, stm);
     b->d_rec_beg.upload(rec_beg, stm);
+    b->rec_group = ordered_group(rec_beg);
     if (rec.empty()) rec.push_back(Tap{});
     b->d_rec.upload(rec, stm);
     b->d_rec_w.upload(rec_w, stm);
@@ -1184,22 +1195,26 @@ void run_forward2(owl_elastic2d* b, bool save_boundary) {
     const unsigned nshot = unsigned(b->sd.size());
     double bs, bv;
     sweep_bytes2(b, bs, bv);
-    const unsigned rg = unsigned(std::max(1, (2 * b->max_nr + 255) / 256));
+    const unsigned rg = unsigned(std::max(1, (2 * b->max_nr + b->rec_group - 1) / b->rec_group));
     // step t: [boundary record of the state at the start of the step] ->
     // record(t) -> update -> source (submodule_forward_modeling.f90:31-180)
     auto loop = [&] {
         for (int t = 1; t <= b->nt; ++t) {
             if (save_boundary) strips2(b, F.vx, F.vz, t, 1);
             int ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(k2e_record, dim3(rg, nshot), dim3(256), 0, st, b->d_shots.get(), F.vx, F.vz,
-                               b->d_rec_beg.get(), b->d_rec.get(), b->d_rec_w.get(), b->d_traces.get(), b->nt, t);
+            hipLaunchKernelGGL(k2e_record, dim3(rg, nshot), dim3(kOrderedThreads), 0, st, b->d_shots.get(), F.vx, F.vz,
+                               b->d_rec_beg.get(), b->d_rec.get(), b->d_rec_w.get(), b->d_traces.get(), b->nt, t,
+                               b->rec_group);
             b->prof.end(st, ev);
             if (t == b->nt) break;  // the last update changes nothing that is recorded
             step2<R>(b, F, out_of(F), b->dt, bs, bv);
-            ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(k2e_inject, dim3(nshot), dim3(1024), 0, st, b->d_shots.get(), F.vx, F.vz, F.sxx,
-                               F.szz, b->d_inj_beg.get(), b->d_inj.get(), b->d_amp.get(), b->nt, t);
-            b->prof.end(st, ev);
+            // outside every source's active steps the injection would change nothing
+            if (t >= b->src_t0 && t <= b->src_t1) {
+                ev = b->prof.begin(st, 2, 0);
+                hipLaunchKernelGGL(k2e_inject, dim3(nshot), dim3(1024), 0, st, b->d_shots.get(), F.vx, F.vz, F.sxx,
+                                   F.szz, b->d_inj_beg.get(), b->d_inj.get(), b->d_amp.get(), b->nt, t);
+                b->prof.end(st, ev);
+            }
             if (!b->graph.capturing) maybe_collect(b);
         }
     };

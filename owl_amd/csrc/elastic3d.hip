@@ -19,6 +19,7 @@
 
 #include "common.hpp"
 #include "host_prep.hpp"
+#include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
 #include "record_store.hpp"
@@ -543,40 +544,35 @@ __global__ __launch_bounds__(1024) void ke_inject(const ShotE* __restrict__ shot
 }
 
 // Receivers of step t: vx at (hx, gy, gz), vy at (gx, hy, gz), vz at
-// (gx, gy, hz) (submodule_forward_modeling.f90:75-140).  The taps of a box
-// are summed z, y, x outermost to innermost, skipping zero weights, as OWL
-// lists them.
-__global__ __launch_bounds__(256) void ke_record(const ShotE* __restrict__ shots, EF F,
-                                                 const RecBox* __restrict__ boxes,
-                                                 const float* __restrict__ rec_w, float* traces, int nt, int t) {
+// (gx, gy, hz) (submodule_forward_modeling.f90:75-140), kRecGroup of a
+// shot's 3 nr components to a block.  The taps of a box are summed z, y, x
+// outermost to innermost as OWL lists them; a tap of zero weight, which OWL
+// leaves out, adds +0 (its cell may lie outside the grid and is not read).
+constexpr int kBoxTaps = (2 * kNkw + 1) * (2 * kNkw + 1) * (2 * kNkw + 1);
+constexpr int kRecGroup = kOrderedTaps / kBoxTaps;
+
+__global__ __launch_bounds__(kOrderedThreads) void ke_record(const ShotE* __restrict__ shots, EF F,
+                                                             const RecBox* __restrict__ boxes,
+                                                             const float* __restrict__ rec_w, float* traces, int nt,
+                                                             int t) {
     constexpr int K = 2 * kNkw + 1;
     const ShotE S = shots[blockIdx.y];
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < 3 * S.nr; r += gridDim.x * blockDim.x) {
-        const int comp = r / S.nr, ir = r % S.nr;
-        const RecBox& B = boxes[3 * S.rec0 + comp * S.nr + ir];
-        const float w = rec_w[S.rec0 + ir];
-        const float* f = comp == 0 ? F.vx : (comp == 1 ? F.vy : F.vz);
-        float wx[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) wx[k] = B.w[0][k];
-        float acc = 0.0f;
-        for (int kz = 0; kz < K; ++kz) {
-            const float w3 = B.w[2][kz];
-            if (w3 == 0.f) continue;
-            for (int ky = 0; ky < K; ++ky) {
-                const float w2 = B.w[1][ky];
-                if (w2 == 0.f) continue;
-                const float* row = f + (B.cell0 + (long long)ky * S.px + (long long)kz * S.pxy);
-#pragma unroll
-                for (int kx = 0; kx < K; ++kx) {
-                    const float w1 = wx[kx];
-                    if (w1 == 0.f) continue;
-                    acc = acc + row[kx] * w1 * w2 * w3 * w;
-                }
-            }
-        }
-        traces[S.trace0 + size_t(comp) * nt * S.nr + size_t(t - 1) * S.nr + ir] = acc;
-    }
+    const int r0 = int(blockIdx.x) * kRecGroup, r1 = min(r0 + kRecGroup, 3 * S.nr);
+    ordered_sums(
+        r0, r1, [](int r) { return r * kBoxTaps; },
+        [&](int k) {
+            const int r = k / kBoxTaps, o = k % kBoxTaps;
+            const int kz = o / (K * K), ky = o / K % K, kx = o % K;
+            const RecBox& B = boxes[3 * S.rec0 + r];
+            const float w1 = B.w[0][kx], w2 = B.w[1][ky], w3 = B.w[2][kz];
+            if (w1 == 0.f || w2 == 0.f || w3 == 0.f) return 0.0f;
+            const float* f = r < S.nr ? F.vx : (r < 2 * S.nr ? F.vy : F.vz);
+            return f[B.cell0 + kx + (long long)ky * S.px + (long long)kz * S.pxy] * w1 * w2 * w3;
+        },
+        [](int) { return 0.0f; }, [&](int r) { return rec_w[S.rec0 + r % S.nr]; },
+        [&](int r, float acc) {
+            traces[S.trace0 + size_t(r / S.nr) * nt * S.nr + size_t(t - 1) * S.nr + r % S.nr] = acc;
+        });
 }
 
 // ---------------------------------------------------------------------------
@@ -884,6 +880,7 @@ struct owl_elastic3d {
     DevBuf<float> med[9];   // c11, c12, mu_yz, mu_xz, mu_xy, rho_x, rho_y, rho_z, c44 at the nodes
     DevBuf<float> fld[27];  // nine wavefields, eighteen memory variables
     DevBuf<Tap> d_inj;
+    int src_t0 = 1, src_t1 = 0;    // steps during which any source tap is active
     DevBuf<RecBox> d_rec_box;
     // gradient: boundary records, the other half of the reverse ping-pong,
     // the adjoint field, adjoint-source CSR, accumulators
@@ -985,6 +982,8 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
     std::vector<int> adj_beg{0};
     std::vector<Tap> adj_taps;
     b->max_nadj = 0;
+    b->src_t0 = 1 << 30;
+    b->src_t1 = -1;
     for (int s = 0; s < nshot; ++s) {
         const owl_shot& in = shots[s];
         ShotHostE& H = b->hs[s];
@@ -1085,6 +1084,8 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
                 S.hnt = std::max(hnt, 1);
             }
             const int nbeg = fortran_nint(sc.t0 / cfg->dt) + 1, nend = nbeg + int(stf.size()) - 1;
+            b->src_t0 = std::min(b->src_t0, nbeg);
+            b->src_t1 = std::max(b->src_t1, nend);
             if (sc.mechanism == OWL_EXPLOSION) {
                 const int row = int(amp.size() / nt);
                 for (int t = 1; t <= nt; ++t) {
@@ -1399,7 +1400,7 @@ void run_forward_e(owl_elastic3d* b, bool save_boundary) {
     const unsigned nshot = unsigned(b->sd.size());
     double bs, bv;
     sweep_bytes(b, bs, bv);
-    const unsigned rg = unsigned(std::max(1, (3 * b->max_nr + 255) / 256));
+    const unsigned rg = unsigned(std::max(1, (3 * b->max_nr + kRecGroup - 1) / kRecGroup));
     // step t: [boundary record of the state at the start of the step] ->
     // [free surface: mirror v above it] -> record(t) -> update -> source
     auto loop = [&] {
@@ -1408,7 +1409,7 @@ void run_forward_e(owl_elastic3d* b, bool save_boundary) {
             if (b->fs)
                 hipLaunchKernelGGL(ke_surface<R>, dim3(256, nshot), dim3(256), 0, st, b->d_shots.get(), F, b->pml, 2);
             int ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(ke_record, dim3(rg, nshot), dim3(256), 0, st, b->d_shots.get(), F, b->d_rec_box.get(),
+            hipLaunchKernelGGL(ke_record, dim3(rg, nshot), dim3(kOrderedThreads), 0, st, b->d_shots.get(), F, b->d_rec_box.get(),
                                b->d_rec_w.get(), b->d_traces.get(), b->nt, t);
             b->prof.end(st, ev);
             if (t == b->nt) {
@@ -1422,10 +1423,13 @@ void run_forward_e(owl_elastic3d* b, bool save_boundary) {
                 break;
             }
             step_e<R>(b, F, out_of(F), b->dt, bs, bv);
-            ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(ke_inject, dim3(nshot), dim3(1024), 0, st, b->d_shots.get(), F, b->d_inj_beg.get(),
-                               b->d_inj.get(), b->d_amp.get(), b->nt, t);
-            b->prof.end(st, ev);
+            // outside every source's active steps the injection would change nothing
+            if (t >= b->src_t0 && t <= b->src_t1) {
+                ev = b->prof.begin(st, 2, 0);
+                hipLaunchKernelGGL(ke_inject, dim3(nshot), dim3(1024), 0, st, b->d_shots.get(), F, b->d_inj_beg.get(),
+                                   b->d_inj.get(), b->d_amp.get(), b->nt, t);
+                b->prof.end(st, ev);
+            }
             if (!b->graph.capturing) maybe_collect(b);
         }
     };

@@ -34,6 +34,7 @@
 #include "common.hpp"
 #include "fs_mesh.hpp"
 #include "host_prep.hpp"
+#include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
 #include "record_store.hpp"
@@ -109,6 +110,15 @@ struct Tap {
     int row;
     int tbeg, tend;
     int field;  // 0 vx_hi, 1 vz_hi, 2 vx_ih, 3 vz_ih, 4 sxx_ii, 5 szz_ii, 6 sxx_hh, 7 szz_hh
+};
+
+// One receiver tap, as the sampling reads it: the element (fields stay below
+// 2^29 elements) with the sub-grid in the top bit (0 hi, 1 ih), and w1 w2
+// weight 0.5.  A quarter of a Tap's bytes: the taps are the sampling's
+// largest stream.
+struct RecTapF {
+    unsigned at;
+    float w;
 };
 
 struct Targets {
@@ -616,20 +626,23 @@ __global__ __launch_bounds__(1024) void k_fsg_inject(const ShotF* __restrict__ s
 // Receivers of step t: for each stencil tap (irz, irx), vx_hi at (hx, gz)
 // times amp1 then vx_ih at (gx, hz) times amp2, amp = w1 w2 weight 0.5
 // (submodule_forward_modeling.f90:78-118); likewise vz.
-__global__ __launch_bounds__(256) void k_fsg_record(const ShotF* __restrict__ shots, Targets T,
-                                                    const int* __restrict__ rec_beg, const Tap* __restrict__ rec,
-                                                    float* traces, int nt, int t) {
+// `group` receivers of a shot to a block.
+__global__ __launch_bounds__(kOrderedThreads) void k_fsg_record(const ShotF* __restrict__ shots, Targets T,
+                                                                const int* __restrict__ rec_beg,
+                                                                const RecTapF* __restrict__ rec, float* traces,
+                                                                int nt, int t, int group) {
     const ShotF S = shots[blockIdx.y];
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < 2 * S.nr; r += gridDim.x * blockDim.x) {
-        const int comp = r / S.nr, ir = r % S.nr;
-        const int g = S.rec0 + ir;
-        float acc = 0.0f;
-        for (int k = rec_beg[g]; k < rec_beg[g + 1]; ++k) {
-            const Tap tp = rec[k];  // field 0 (hi grid) or 2 (ih grid)
-            acc = acc + T.f[tp.field + comp][tp.cell] * tp.w;
-        }
-        traces[S.trace0 + size_t(comp) * nt * S.nr + size_t(t - 1) * S.nr + ir] = acc;
-    }
+    // a receiver's taps serve both components: blockIdx.z is the component
+    const int r0 = int(blockIdx.x) * group, r1 = min(r0 + group, S.nr), comp = int(blockIdx.z);
+    const float *hi = T.f[comp], *ih = T.f[2 + comp];
+    ordered_sums(
+        r0, r1, [&](int r) { return rec_beg[S.rec0 + r]; },
+        [&](int k) {
+            const RecTapF tp = rec[k];
+            return ((tp.at >> 31) ? ih : hi)[tp.at & 0x7fffffffu] * tp.w;
+        },
+        [](int) { return 0.0f; }, [](int) { return 1.0f; },
+        [&](int r, float acc) { traces[S.trace0 + size_t(comp) * nt * S.nr + size_t(t - 1) * S.nr + r] = acc; });
 }
 
 // Boundary records (module_boundary_saving.f90:100-200): vx_hi, vz_hi,
@@ -827,7 +840,10 @@ struct owl_fsg2d {
     DevBuf<float> fld[kNF];
     DevBuf<float> fB[kNW];  // the other half of the reverse ping-pong
     DevBuf<float> aF[kNF];  // adjoint field
-    DevBuf<Tap> d_inj, d_rec, d_adj_taps;
+    DevBuf<Tap> d_inj, d_adj_taps;
+    DevBuf<RecTapF> d_rec;
+    int rec_group = 1;                 // receivers per block of the sampling
+    int src_t0 = 1, src_t1 = 0;        // steps during which any source tap is active
     DevBuf<double> d_g[7], d_full, d_misfit, d_scratch;
     // the forward time loop as one HIP graph (modelling without profiling
     // or boundary records), re-captured when a launch argument changes
@@ -1037,6 +1053,8 @@ void planf(owl_fsg2d* b, const owl_acoustic_config* cfg, const float* const* cij
     b->hs.assign(nshot, ShotHostF{});
     b->sd.assign(nshot, ShotF{});
     b->nrec_total = b->max_nr = b->max_nadj = 0;
+    b->src_t0 = 1 << 30;
+    b->src_t1 = -1;
     b->pts_full = 0;
     long long off = 0, trace = 0, strip = 0, grad = 0, out = 0;
     std::vector<float> amp, rec_w;
@@ -1150,6 +1168,8 @@ void planf(owl_fsg2d* b, const owl_acoustic_config* cfg, const float* const* cij
                 S.hnt = std::max(hnt, 1);
             }
             const int nbeg = fortran_nint(sc.t0 / cfg->dt) + 1, nend = nbeg + int(stf.size()) - 1;
+            b->src_t0 = std::min(b->src_t0, nbeg);
+            b->src_t1 = std::max(b->src_t1, nend);
             // with the free surface only rows >= 2 take the source (add_source)
             auto taps = [&](int gx, int gz, const float* wx, const float* wz, int field, int row) {
                 for (int irz = -kNkw; irz <= kNkw; ++irz)
@@ -1285,9 +1305,9 @@ void planf(owl_fsg2d* b, const owl_acoustic_config* cfg, const float* const* cij
     retilef(b);
     damping_ratios(b);
     std::vector<int> rec_beg{0};
-    std::vector<Tap> rec;
+    std::vector<RecTapF> rec;
     for (auto& v : rec_taps) {
-        rec.insert(rec.end(), v.begin(), v.end());
+        for (const Tap& tp : v) rec.push_back(RecTapF{unsigned(tp.cell) | (tp.field ? 0x80000000u : 0u), tp.w});
         rec_beg.push_back(int(rec.size()));
     }
     if (!b->stream) {
@@ -1304,7 +1324,8 @@ void planf(owl_fsg2d* b, const owl_acoustic_config* cfg, const float* const* cij
     if (inj.empty()) inj.push_back(Tap{});
     b->d_inj.upload(inj, stm);
     b->d_rec_beg.upload(rec_beg, stm);
-    if (rec.empty()) rec.push_back(Tap{});
+    b->rec_group = ordered_group(rec_beg);
+    if (rec.empty()) rec.push_back(RecTapF{});
     b->d_rec.upload(rec, stm);
     b->d_rec_w.upload(rec_w, stm);
     b->d_adj_beg.upload(adj_beg, stm);
@@ -1613,22 +1634,25 @@ void run_forwardf(owl_fsg2d* b, bool save_boundary) {
     const unsigned nshot = unsigned(b->sd.size());
     double bs, bv;
     sweep_bytesf(b, bs, bv);
-    const unsigned rg = unsigned(std::max(1, (2 * b->max_nr + 255) / 256));
+    const unsigned rg = unsigned(std::max(1, (b->max_nr + b->rec_group - 1) / b->rec_group));
     // step t: [boundary record] -> record(t) -> update -> source(t)
     // (submodule_forward_modeling.f90:55-240)
     auto loop = [&] {
         for (int t = 1; t <= b->nt; ++t) {
             if (save_boundary) stripsf(b, V, t, 1);
             int ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(k_fsg_record, dim3(rg, nshot), dim3(256), 0, st, b->d_shots.get(), vel_targets(V),
-                               b->d_rec_beg.get(), b->d_rec.get(), b->d_traces.get(), b->nt, t);
+            hipLaunchKernelGGL(k_fsg_record, dim3(rg, nshot, 2), dim3(kOrderedThreads), 0, st, b->d_shots.get(), vel_targets(V),
+                               b->d_rec_beg.get(), b->d_rec.get(), b->d_traces.get(), b->nt, t, b->rec_group);
             b->prof.end(st, ev);
             if (t == b->nt) break;  // the last update changes nothing that is recorded
             stepf<R>(b, F, V, b->dt, bs, bv);
-            ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(k_fsg_inject, dim3(nshot), dim3(1024), 0, st, b->d_shots.get(), vel_targets(V),
-                               b->d_inj_beg.get(), b->d_inj.get(), b->d_amp.get(), b->nt, t);
-            b->prof.end(st, ev);
+            // outside every source's active steps the injection would change nothing
+            if (t >= b->src_t0 && t <= b->src_t1) {
+                ev = b->prof.begin(st, 2, 0);
+                hipLaunchKernelGGL(k_fsg_inject, dim3(nshot), dim3(1024), 0, st, b->d_shots.get(), vel_targets(V),
+                                   b->d_inj_beg.get(), b->d_inj.get(), b->d_amp.get(), b->nt, t);
+                b->prof.end(st, ev);
+            }
             if (!b->graph.capturing) maybe_collectf(b);
         }
     };
