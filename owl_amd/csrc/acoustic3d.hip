@@ -20,6 +20,7 @@
 
 #include "common.hpp"
 #include "host_prep.hpp"
+#include "launch_shape.hpp"
 #include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
@@ -1549,11 +1550,11 @@ using namespace owl::a3;
 
 struct owl_acoustic3d {
     owl_acoustic_config cfg{};
-    int R = 4, pml = 15, nt = 0, kc = 64;
-    int variant = 1;   // 0: LDS planes with barriers, 1: barrier-free columns, 2: four-wide, 3: pipelined columns
+    int R = 4, pml = 15, nt = 0, kc = 0;  // kc: planes per tile, set by the plan if 0
+    int variant = 2;   // 0: LDS planes with barriers, 1: barrier-free columns, 2: four-wide, 3: pipelined columns
     int cy = 4;        // rows per block of the column variant
-    int remap = 0;     // XCD-contiguous tile order
-    int launch_code = 1;  // the public variant code of the current shape
+    int remap = 1;     // XCD-contiguous tile order
+    int launch_code = 24;  // the public variant code of the current shape
     bool fused = false;   // forward steps by the fused kernel (k3f_step; no free surface)
     int fkc = 64;         // z planes per tile of the fused kernel
     std::vector<int> ftile_shot;
@@ -1659,6 +1660,13 @@ void fused_shape(int R, int& W, int& TY) {
 void retile(owl_acoustic3d* b) {
     const int pml = b->pml;
     b->tile_shot.clear();
+    if (b->kc < 1) {
+        double waves = 0;
+        for (const Shot3& S : b->sd)
+            waves += double((S.nx + 2 * pml + 4 * kWX - 1) / (4 * kWX)) * double(S.ny + 2 * pml) *
+                     double(S.nz + (b->fs ? 1 : 2) * pml) * (kWX / 64.0);
+        b->kc = default_planes(waves);
+    }
     const int ty_rows = b->variant == 0 ? kTY : (b->variant == 2 ? kWY : b->cy);
     const int tx_cols = b->variant == 2 ? 4 * kWX : kBX;
     for (size_t s = 0; s < b->sd.size(); ++s) {
@@ -2334,9 +2342,9 @@ void set_shape(owl_acoustic3d* b, int planes, int variant);
 // does not depend on the field values.
 template <int R>
 void autotune3(owl_acoustic3d* b, int steps) {
-    static const int kVariants[] = {1, 2, 3, 5, 6, 8, 24, 9, 10, 11, 13, 0};
-    static const int kPlanes[] = {32, 64, 128};
-    static const int kFusedPlanes[] = {32, 64, 96, 128, 192};
+    static const int kVariants[] = {24, 8, 5, 13};
+    static const int kPlanes[] = {2, 4, 8, 16, 32};
+    static const int kFusedPlanes[] = {64, 192};
     hipStream_t st = b->stream;
     for (auto& x : b->f) x.zero(st);
     for (auto& x : b->m) x.zero(st);

@@ -24,6 +24,7 @@
 #include "common.hpp"
 #include "fs_mesh.hpp"
 #include "host_prep.hpp"
+#include "launch_shape.hpp"
 #include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
@@ -536,7 +537,7 @@ struct owl_elastic2d {
     float fs_refine = 4.0f, fs_dzmax = 0.0f;
     std::vector<owl::fsm::SsgMesh> mesh;   // per shot (free surface)
     std::vector<std::vector<float>> rho_map;  // per shot: rho on the refined rows, column i (1..nx) at [(i-1) nrj + j + pml]
-    int R = 4, pml = 15, nt = 0, kc = 32, cy = 4;
+    int R = 4, pml = 15, nt = 0, kc = 0, cy = 4;  // kc: rows per tile, set by the plan if 0
     float dt = 0, idx = 0, idz = 0;
     e2::Coef coef{};
     std::vector<ShotHostE2> hs;
@@ -649,6 +650,13 @@ void damp_axis_rows(int n, int pml, const std::vector<float>& dzi, float pmlvp, 
 
 void retile2(owl_elastic2d* b) {
     b->tile_shot.clear();
+    if (b->kc < 1) {
+        double waves = 0;
+        for (const ShotE2& S : b->sd)
+            waves += double((S.nx + 2 * b->pml + (64 - 2 * b->R) - 1) / (64 - 2 * b->R)) *
+                     double(S.nz + (b->fs ? 1 : 2) * b->pml);
+        b->kc = default_planes(waves);
+    }
     for (size_t s = 0; s < b->sd.size(); ++s) {
         ShotE2& S = b->sd[s];
         S.ntx = (S.nx + 2 * b->pml + (64 - 2 * b->R) - 1) / (64 - 2 * b->R);  // sweeps update 64 - 2R columns
@@ -1579,7 +1587,7 @@ owl_status owl_elastic2d_set_graphs(owl_elastic2d* b, int on) {
 owl_status owl_elastic2d_autotune(owl_elastic2d* b, int steps, int* planes, int* rows) {
     return guarded([&] {
         if (!b || steps < 1) fail(OWL_ERR_ARG, "null batch or no steps");
-        static const int kPlanes[] = {4, 8, 12, 16, 32, 64, 128};
+        static const int kPlanes[] = {4, 8, 12, 16, 32};
         static const int kRows[] = {1, 2, 4};
         hipStream_t st = b->stream;
         const bool prof_on = b->prof.on();

@@ -19,6 +19,7 @@
 
 #include "common.hpp"
 #include "host_prep.hpp"
+#include "launch_shape.hpp"
 #include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
@@ -859,7 +860,7 @@ using namespace owl::e3;
 
 struct owl_elastic3d {
     owl_acoustic_config cfg{};
-    int R = 4, pml = 15, nt = 0, kc = 64, cy = kCY, fs = 0;
+    int R = 4, pml = 15, nt = 0, kc = 0, cy = kCY, fs = 0;  // kc: planes per tile, set by the plan if 0
     float dt = 0, idx = 0, idy = 0, idz = 0;
     e3::Coef coef{};
     std::vector<ShotHostE> hs;
@@ -942,6 +943,29 @@ void mpml_axis(int n, int pml, float d, float pmlvp, float alphamax, bool top_of
     for (auto* v : {&di, &dh, &ai, &ah}) out.insert(out.end(), v->begin(), v->end());
 }
 
+void retile_e(owl_elastic3d* b) {
+    int lt = 0;
+    b->tile_shot.clear();
+    if (b->kc < 1) {
+        double waves = 0;
+        for (const ShotE& S : b->sd)
+            waves += double((S.nx + 2 * b->pml + (64 - 2 * b->R) - 1) / (64 - 2 * b->R)) * double(S.ny + 2 * b->pml) *
+                     double(S.nz + (b->fs ? 1 : 2) * b->pml);
+        b->kc = default_planes(waves);
+    }
+    for (size_t s = 0; s < b->sd.size(); ++s) {
+        ShotE& S = b->sd[s];
+        S.nty = (S.ny + 2 * b->pml + b->cy - 1) / b->cy;
+        S.ntx = (S.nx + 2 * b->pml + (64 - 2 * b->R) - 1) / (64 - 2 * b->R);
+        S.nzc = (S.nz + 2 * b->pml + b->kc - 1) / b->kc;
+        S.tile0 = lt;
+        lt += S.ntx * S.nty * S.nzc;
+        b->tile_shot.insert(b->tile_shot.end(), size_t(S.ntx) * S.nty * S.nzc, int(s));
+    }
+    b->d_shots.upload(b->sd, b->stream);
+    b->d_tile_shot.upload(b->tile_shot, b->stream);
+}
+
 void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, const float* vs, const float* rho,
             int nshot, const owl_shot* shots) {
     if (!cfg || !vp || !vs || !rho || nshot < 1 || !shots) fail(OWL_ERR_ARG, "null argument or no shots");
@@ -970,7 +994,6 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
     const int R = b->R, pml = b->pml, nt = b->nt, lo = 1 - pml - R;
     b->hs.assign(nshot, ShotHostE{});
     b->sd.assign(nshot, ShotE{});
-    b->tile_shot.clear();
     b->nrec_total = b->max_nr = 0;
     b->pts_full = 0;
     long long off = 0, trace = 0, strip = 0, grad = 0;
@@ -1035,11 +1058,6 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
         S.off = off;
         off += S.pxy * S.nzp;
         off = (off + 63) / 64 * 64;
-        S.nty = (H.ny + 2 * pml + b->cy - 1) / b->cy;
-        S.ntx = (H.nx + 2 * pml + (64 - 2 * R) - 1) / (64 - 2 * R);  // sweeps update 64 - 2R columns per wavefront
-        S.nzc = (H.nz + 2 * pml + b->kc - 1) / b->kc;
-        S.tile0 = int(b->tile_shot.size());
-        b->tile_shot.insert(b->tile_shot.end(), size_t(S.ntx) * S.nty * S.nzc, s);
         b->pts_full += double(H.nx + 2 * pml) * double(H.ny + 2 * pml) * double(H.nz + 2 * pml);
         S.prof = prof;
         const float amax = float(double(1.0f * f0max) * M_PI);
@@ -1223,8 +1241,7 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
         OWL_HIP(hipEventCreate(&b->ev1));
     }
     hipStream_t stm = b->stream;
-    b->d_shots.upload(b->sd, stm);
-    b->d_tile_shot.upload(b->tile_shot, stm);
+    retile_e(b);
     b->d_prof.upload(profs, stm);
     if (amp.empty()) amp.push_back(0.f);
     b->d_amp.upload(amp, stm);
@@ -1598,22 +1615,6 @@ inline void chain_rule(float vp, float vs, float rho, double A, double B, double
 
 // Tiles of the current launch shape (kc z planes, cy y rows per tile) and
 // their shots, uploaded on the batch's stream.
-void retile_e(owl_elastic3d* b) {
-    int lt = 0;
-    b->tile_shot.clear();
-    for (size_t s = 0; s < b->sd.size(); ++s) {
-        ShotE& S = b->sd[s];
-        S.nty = (S.ny + 2 * b->pml + b->cy - 1) / b->cy;
-        S.ntx = (S.nx + 2 * b->pml + (64 - 2 * b->R) - 1) / (64 - 2 * b->R);
-        S.nzc = (S.nz + 2 * b->pml + b->kc - 1) / b->kc;
-        S.tile0 = lt;
-        lt += S.ntx * S.nty * S.nzc;
-        b->tile_shot.insert(b->tile_shot.end(), size_t(S.ntx) * S.nty * S.nzc, int(s));
-    }
-    b->d_shots.upload(b->sd, b->stream);
-    b->d_tile_shot.upload(b->tile_shot, b->stream);
-}
-
 }  // namespace
 
 extern "C" {
@@ -1748,7 +1749,7 @@ owl_status owl_elastic3d_set_launch(owl_elastic3d* b, int planes, int rows) {
 owl_status owl_elastic3d_autotune(owl_elastic3d* b, int steps, int* planes, int* rows) {
     return guarded([&] {
         if (!b || steps < 1) fail(OWL_ERR_ARG, "null batch or no steps");
-        static const int kPlanes[] = {8, 12, 16, 32, 64, 128, 256};
+        static const int kPlanes[] = {8, 12, 16, 32};
         static const int kRows[] = {1, 2, 4};
         hipStream_t st = b->stream;
         const bool prof_on = b->prof.on();

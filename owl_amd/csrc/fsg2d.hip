@@ -34,6 +34,7 @@
 #include "common.hpp"
 #include "fs_mesh.hpp"
 #include "host_prep.hpp"
+#include "launch_shape.hpp"
 #include "ordered_sum.hpp"
 #include "owl_amd.h"
 #include "profiler.hpp"
@@ -811,7 +812,7 @@ using namespace owl::fsg;
 
 struct owl_fsg2d {
     owl_acoustic_config cfg{};
-    int R = 4, pml = 15, nt = 0, kc = 32, cy = 4, aniso = 1, restore_all = 0;
+    int R = 4, pml = 15, nt = 0, kc = 0, cy = 4, aniso = 1, restore_all = 0;  // kc: rows per tile, set by the plan if 0
     float dt = 0;
     bool fs = false;  // OWL's free surface on the refined mesh
     fsm::Surface surf;
@@ -960,6 +961,13 @@ void damping_ratios(owl_fsg2d* b) {
 
 void retilef(owl_fsg2d* b) {
     b->tile_shot.clear();
+    if (b->kc < 1) {
+        double waves = 0;
+        for (const ShotF& S : b->sd)
+            waves += double((S.nx + 2 * b->pml + (64 - 2 * b->R) - 1) / (64 - 2 * b->R)) *
+                     double(S.nz + (b->fs ? 1 : 2) * b->pml);
+        b->kc = default_planes(waves);
+    }
     for (size_t s = 0; s < b->sd.size(); ++s) {
         ShotF& S = b->sd[s];
         const int W = 64 - 2 * b->R;  // columns a tile updates (the sweeps' halo lanes feed shuffles)
@@ -2058,7 +2066,7 @@ owl_status owl_fsg2d_set_graphs(owl_fsg2d* b, int on) {
 owl_status owl_fsg2d_autotune(owl_fsg2d* b, int steps, int* planes, int* rows) {
     return guarded([&] {
         if (!b || steps < 1) fail(OWL_ERR_ARG, "null batch or no steps");
-        static const int kPlanes[] = {4, 8, 12, 16, 32, 64, 128};
+        static const int kPlanes[] = {4, 8, 12, 16, 32};
         static const int kRows[] = {1, 2, 4};
         hipStream_t st = b->stream;
         const bool prof_on = b->prof.on();

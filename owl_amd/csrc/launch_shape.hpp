@@ -1,0 +1,27 @@
+// Default launch shape of the marching sweeps.
+#pragma once
+
+namespace owl {
+
+// Rows (2D) or planes (3D) that one wavefront marches over, from the number
+// of wavefronts the batch has at one row or plane each.  A wavefront's march
+// is serial, a few us a row when few wavefronts share a SIMD, so a small
+// batch wants as many wavefronts as it can have; a large one wants longer
+// marches, whose fill of the z queue (2R rows) weighs less.  The line is
+// where the chip holds about twice the wavefronts that run at once.
+// us per step on one MI355X at 2 / 4 / 8 / 32 rows: 2D elastic 301 x 201,
+// 1 shot 19 / 27 / 43 / 136, 8 shots 34 / 41 / 58 / 161, 32 shots 92 / 86 /
+// 84 / 188; FSG 333 x 171, 8 shots 58 / 59 / 81 / 227; 801 x 401, 32 shots
+// 723 / 688 / 687 / 783; 3D elastic 50 x 45 x 40 79 / 78 / 109 / 300, 117 x
+// 90 x 75, 2 shots 342 / 343 / 361 / 497; 200 x 200 x 150, 4 shots 3054 /
+// 2905 / 2891 / 3090; 3D acoustic (four-wide columns) 50 x 45 x 40 24 / 27 /
+// 39 / 106, 121 x 110 x 93, 2 shots 105 / 102 / 110 / 149, 256^3, 16 shots
+// 4499 / 4264 / 4203 / 4458.
+inline int default_planes(double wavefronts) {
+    constexpr double kEnough = 14000.0;
+    if (wavefronts / 8 >= kEnough) return 8;
+    if (wavefronts / 4 >= kEnough) return 4;
+    return 2;
+}
+
+}  // namespace owl
