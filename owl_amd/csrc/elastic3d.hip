@@ -94,20 +94,6 @@ __device__ __forceinline__ size_t ate(const ShotE& S, int lo, int i, int j, int 
     return size_t(S.off) + size_t(i - lo) + size_t(j - lo) * size_t(S.px) + size_t(k - lo) * size_t(S.pxy);
 }
 
-// damp_coef + damp_wavefield (module_wavefield.f90:40-47) with kappa = 1.
-// A node whose own-axis profile is zero keeps a zero memory variable and an
-// unchanged derivative, so the update is skipped there.
-__device__ __forceinline__ float damp(float* w, size_t q, float v, float d, float alpha, float adt) {
-    if (d == 0.0f) return v;
-    const float a_ = d / 1.0f;
-    const float b_ = d / 1.0f + alpha;
-    const float ca = -(2.0f * adt * a_ / (2.0f + adt * b_));
-    const float cb = (2.0f - adt * b_) / (2.0f + adt * b_);
-    const float m = ca * v + cb * w[q];
-    w[q] = m;
-    return (v + m) / 1.0f;
-}
-
 // Load and store at a 32-bit byte offset from a kernel-argument base (the
 // sweeps' fields stay below 2 GiB, checked on the host): every array of a
 // sweep is addressed by a few shared offset registers against scalar bases.
@@ -117,15 +103,18 @@ __device__ __forceinline__ float ldo(const float* base, unsigned off) {
 __device__ __forceinline__ void sto(float* base, unsigned off, float v) {
     *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + off) = v;
 }
-__device__ __forceinline__ float damp_o(float* w, unsigned qb, float v, float d, float alpha, float adt) {
-    if (d == 0.0f) return v;
-    const float a_ = d / 1.0f;
-    const float b_ = d / 1.0f + alpha;
-    const float ca = -(2.0f * adt * a_ / (2.0f + adt * b_));
-    const float cb = (2.0f - adt * b_) / (2.0f + adt * b_);
-    const float m = ca * v + cb * ldo(w, qb);
-    sto(w, qb, m);
-    return (v + m) / 1.0f;
+// damp_coef + damp_wavefield (module_wavefield.f90:40-47) with kappa = 1:
+// memory variable m = a v + b m, derivative v + m.  a, b come from the
+// profiles (mpml_axis); a node whose own-axis damping is zero (a = 0) keeps
+// a zero memory variable and an unchanged derivative, so nothing is loaded
+// or stored there.  The old m is loaded ahead of its use (mem_o): loaded
+// where it is used, every damped derivative waited for its own round trip
+// to memory, since no load moves up over the store before it.
+__device__ __forceinline__ float mem_o(const float* w, unsigned qb, bool on) { return on ? ldo(w, qb) : 0.0f; }
+__device__ __forceinline__ float damp_o(float* w, unsigned qb, float v, float a, float b, float m0, bool on) {
+    const float m = a * v + b * m0;
+    if (on) sto(w, qb, m);
+    return on ? v + m : v;
 }
 
 // x stencil sum_m c_m (w(i+off+m) - w(i+off-m+1)) from the lanes' values of
@@ -152,8 +141,9 @@ __device__ __forceinline__ float sten_y(const float* w, const unsigned* yo, int 
     return s;
 }
 
+// a and b of the damping at nodes (ai, bi) and half nodes (ah, bh), per axis.
 struct Prof {
-    const float *dix, *dhx, *aix, *ahx, *diy, *dhy, *aiy, *ahy, *diz, *dhz, *aiz, *ahz;
+    const float *aix, *ahx, *bix, *bhx, *aiy, *ahy, *biy, *bhy, *aiz, *ahz, *biz, *bhz;
     int pml;
 };
 
@@ -161,11 +151,11 @@ __device__ __forceinline__ Prof prof_of(const float* prof, const ShotE& S, int p
     const int lx = S.nx + 2 * pml, ly = S.ny + 2 * pml, lz = S.nz + 2 * pml;
     const float* p = prof + S.prof;
     Prof P;
-    P.dix = p; P.dhx = p + lx; P.aix = p + 2 * lx; P.ahx = p + 3 * lx;
+    P.aix = p; P.ahx = p + lx; P.bix = p + 2 * lx; P.bhx = p + 3 * lx;
     p += 4 * lx;
-    P.diy = p; P.dhy = p + ly; P.aiy = p + 2 * ly; P.ahy = p + 3 * ly;
+    P.aiy = p; P.ahy = p + ly; P.biy = p + 2 * ly; P.bhy = p + 3 * ly;
     p += 4 * ly;
-    P.diz = p; P.dhz = p + lz; P.aiz = p + 2 * lz; P.ahz = p + 3 * lz;
+    P.aiz = p; P.ahz = p + lz; P.biz = p + 2 * lz; P.bhz = p + 3 * lz;
     P.pml = pml;
     return P;
 }
@@ -206,7 +196,6 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
     const bool mcol = i <= nx + pml + R;
     const bool own = l >= R && l <= 63 - R && i <= nx + pml;
     const Prof P = prof_of(prof, S, pml);
-    const float adt = fabsf(dt);
     const float* __restrict__ vx = F.vx;
     const float* __restrict__ vy = F.vy;
     const float* __restrict__ vz = F.vz;
@@ -224,6 +213,10 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
     }
     const bool xin = !(i <= 0 || i >= nx + 1), yin = !(j <= 0 || j >= ny + 1);
     const bool Xin = !(i <= 1 || i >= nx + 1), Yin = !(j <= 1 || j >= ny + 1);
+    // damping coefficients of this column and row (0 on lanes that own none)
+    const float aix = own ? P.aix[ii] : 0.0f, bix = own ? P.bix[ii] : 0.0f;
+    const float ahx = own ? P.ahx[ii] : 0.0f, bhx = own ? P.bhx[ii] : 0.0f;
+    const float aiy = P.aiy[jj], biy = P.biy[jj], ahy = P.ahy[jj], bhy = P.bhy[jj];
     // The inputs of one plane: the queues' fronts (plane k + R) and, on the
     // owned lanes, the moduli and old stresses.  Plane k + 1's are loaded
     // while plane k is computed (the y stencils stay direct loads).
@@ -258,12 +251,27 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
         qx[2 * R] = cur.fx;
         qy[2 * R] = cur.fy;
         qz[2 * R] = cur.fz;
+        // the memory variables this plane damps, all in flight together
+        const int kk = k + pml - 1;
+        const float aiz = P.aiz[kk], biz = P.biz[kk], ahz = P.ahz[kk], bhz = P.bhz[kk];
+        const bool top = fs && k == 1, zp0 = (!fs && k <= 0) || k >= nz + 1, zp1 = (!fs && k <= 1) || k >= nz + 1;
+        const bool pn = own && (!xin || !yin || (!top && zp0));       // normal stresses
+        const bool pyz = own && (!xin || !Yin || zp1) && !top, pxz = own && (!Xin || !yin || zp1) && !top;
+        const bool pxy = own && (!Xin || !Yin || (!fs && zp0));
+        const bool d_xvx = pn && aix != 0.0f, d_yvy = pn && aiy != 0.0f, d_zvz = pn && !top && aiz != 0.0f;
+        const bool d_yvz = pyz && ahy != 0.0f, d_zvy = pyz && ahz != 0.0f;
+        const bool d_xvz = pxz && ahx != 0.0f, d_zvx = pxz && ahz != 0.0f;
+        const bool d_xvy = pxy && ahx != 0.0f, d_yvx = pxy && ahy != 0.0f;
+        const float m_xvx = mem_o(F.m_dxvx, q, d_xvx), m_yvy = mem_o(F.m_dyvy, q, d_yvy);
+        const float m_zvz = mem_o(F.m_dzvz, q, d_zvz), m_yvz = mem_o(F.m_dyvz, q, d_yvz);
+        const float m_zvy = mem_o(F.m_dzvy, q, d_zvy), m_xvz = mem_o(F.m_dxvz, q, d_xvz);
+        const float m_zvx = mem_o(F.m_dzvx, q, d_zvx), m_xvy = mem_o(F.m_dxvy, q, d_xvy);
+        const float m_yvx = mem_o(F.m_dyvx, q, d_yvx);
         // x stencils of this plane from the lanes (all lanes take part)
         const float sx_vx = sten_lanes<R>(qx[R], l, 0, c);    // d+x vx
         const float sx_vz = sten_lanes<R>(qz[R], l, -1, c);   // d-x vz
         const float sx_vy = sten_lanes<R>(qy[R], l, -1, c);   // d-x vy
         if (own) {
-            const int kk = k + pml - 1;
             unsigned yo[2 * R + 1];  // rows j - R .. j + R of this plane
 #pragma unroll
             for (int m = 0; m <= 2 * R; ++m) yo[m] = q + unsigned(m - R) * syb;
@@ -271,29 +279,22 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
             {
                 float pdxvx = idx * sx_vx, pdyvy = idy * sten_y<R>(vy, yo, 0, c), pdzvz;
                 const float c11 = cur.c11, c12 = cur.c12;
-                if (fs && k == 1) {
-                    if (!xin || !yin) {
-                        pdxvx = damp_o(F.m_dxvx, q, pdxvx, P.dix[ii], P.aix[ii], adt);
-                        pdyvy = damp_o(F.m_dyvy, q, pdyvy, P.diy[jj], P.aiy[jj], adt);
-                    }
+                pdxvx = damp_o(F.m_dxvx, q, pdxvx, aix, bix, m_xvx, d_xvx);
+                pdyvy = damp_o(F.m_dyvy, q, pdyvy, aiy, biy, m_yvy, d_yvy);
+                if (top) {
                     pdzvz = -(c12 / c11 * pdxvx) - c12 / c11 * pdyvy;
                 } else {
                     float s = c.c[0] * (qz[R + 1] - qz[R]);
 #pragma unroll
                     for (int m = 2; m <= R; ++m) s = s + c.c[m - 1] * (qz[R + m] - qz[R - m + 1]);
-                    pdzvz = idz * s;
-                    if (!xin || !yin || (!fs && k <= 0) || k >= nz + 1) {
-                        pdxvx = damp_o(F.m_dxvx, q, pdxvx, P.dix[ii], P.aix[ii], adt);
-                        pdyvy = damp_o(F.m_dyvy, q, pdyvy, P.diy[jj], P.aiy[jj], adt);
-                        pdzvz = damp_o(F.m_dzvz, q, pdzvz, P.diz[kk], P.aiz[kk], adt);
-                    }
+                    pdzvz = damp_o(F.m_dzvz, q, idz * s, aiz, biz, m_zvz, d_zvz);
                 }
                 sto(O.sxx, q, cur.sxx + dt * (c11 * pdxvx + c12 * pdyvy + c12 * pdzvz));
                 sto(O.syy, q, cur.syy + dt * (c12 * pdxvx + c11 * pdyvy + c12 * pdzvz));
                 sto(O.szz, q, cur.szz + dt * (c12 * pdxvx + c12 * pdyvy + c11 * pdzvz));
             }
             // ---- shear stresses with a z derivative: syz, sxz (Z = k)
-            if (!fs || k >= 2) {
+            if (!top) {
                 float a = c.c[0] * (qy[R] - qy[R - 1]);   // d-z vy
                 float e = c.c[0] * (qx[R] - qx[R - 1]);   // d-z vx
 #pragma unroll
@@ -302,25 +303,18 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
                     e = e + c.c[m - 1] * (qx[R + m - 1] - qx[R - m]);
                 }
                 float pdzvy = idz * a, pdyvz = idy * sten_y<R>(vz, yo, -1, c), pdzvx = idz * e, pdxvz = idx * sx_vz;
-                const bool zpml = (!fs && k <= 1) || k >= nz + 1;
-                if (!xin || !Yin || zpml) {
-                    pdyvz = damp_o(F.m_dyvz, q, pdyvz, P.dhy[jj], P.ahy[jj], adt);
-                    pdzvy = damp_o(F.m_dzvy, q, pdzvy, P.dhz[kk], P.ahz[kk], adt);
-                }
+                pdyvz = damp_o(F.m_dyvz, q, pdyvz, ahy, bhy, m_yvz, d_yvz);
+                pdzvy = damp_o(F.m_dzvy, q, pdzvy, ahz, bhz, m_zvy, d_zvy);
                 sto(O.syz, q, cur.syz + dt * cur.myz * (pdzvy + pdyvz));
-                if (!Xin || !yin || zpml) {
-                    pdxvz = damp_o(F.m_dxvz, q, pdxvz, P.dhx[ii], P.ahx[ii], adt);
-                    pdzvx = damp_o(F.m_dzvx, q, pdzvx, P.dhz[kk], P.ahz[kk], adt);
-                }
+                pdxvz = damp_o(F.m_dxvz, q, pdxvz, ahx, bhx, m_xvz, d_xvz);
+                pdzvx = damp_o(F.m_dzvx, q, pdzvx, ahz, bhz, m_zvx, d_zvx);
                 sto(O.sxz, q, cur.sxz + dt * cur.mxz * (pdzvx + pdxvz));
             }
             // ---- sxy (X, Y, k)
             {
                 float pdyvx = idy * sten_y<R>(vx, yo, -1, c), pdxvy = idx * sx_vy;
-                if (!Xin || !Yin || (!fs && (k <= 0 || k >= nz + 1))) {
-                    pdxvy = damp_o(F.m_dxvy, q, pdxvy, P.dhx[ii], P.ahx[ii], adt);
-                    pdyvx = damp_o(F.m_dyvx, q, pdyvx, P.dhy[jj], P.ahy[jj], adt);
-                }
+                pdxvy = damp_o(F.m_dxvy, q, pdxvy, ahx, bhx, m_xvy, d_xvy);
+                pdyvx = damp_o(F.m_dyvx, q, pdyvx, ahy, bhy, m_yvx, d_yvx);
                 sto(O.sxy, q, cur.sxy + dt * cur.mxy * (pdyvx + pdxvy));
             }
         }
@@ -369,7 +363,6 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
     const bool mcol = i <= nx + pml + R;
     const bool own = l >= R && l <= 63 - R && i <= nx + pml;
     const Prof P = prof_of(prof, S, pml);
-    const float adt = fabsf(dt);
     const float* __restrict__ sxx = O.sxx;
     const float* __restrict__ syy = O.syy;
     const float* __restrict__ szz = O.szz;
@@ -389,6 +382,10 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
     }
     const bool xin = !(i <= 0 || i >= nx + 1), yin = !(j <= 0 || j >= ny + 1);
     const bool Xin = !(i <= 1 || i >= nx + 1), Yin = !(j <= 1 || j >= ny + 1);
+    // damping coefficients of this column and row (0 on lanes that own none)
+    const float aix = own ? P.aix[ii] : 0.0f, bix = own ? P.bix[ii] : 0.0f;
+    const float ahx = own ? P.ahx[ii] : 0.0f, bhx = own ? P.bhx[ii] : 0.0f;
+    const float aiy = P.aiy[jj], biy = P.biy[jj], ahy = P.ahy[jj], bhy = P.bhy[jj];
     // The inputs of one plane: the queues' fronts (plane k + R), sxx and sxy
     // and, on the owned lanes, the densities and old velocities.  Plane
     // k + 1's are loaded while plane k is computed (the y stencils stay
@@ -420,14 +417,26 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
         qa[2 * R] = cur.fa;
         qb[2 * R] = cur.fb;
         qc[2 * R] = cur.fc;
+        // the memory variables this plane damps, all in flight together
+        const int kk = k + pml - 1;
+        const float aiz = P.aiz[kk], biz = P.biz[kk], ahz = P.ahz[kk], bhz = P.bhz[kk];
+        const bool zin = !((!fs && k <= 0) || k >= nz + 1), Zin = !((!fs && k <= 1) || k >= nz + 1);
+        const bool px = own && (!Xin || !yin || !zin), py = own && (!xin || !Yin || !zin);
+        const bool pz = own && (!xin || !yin || !Zin) && (!fs || k >= 2);
+        const bool d_xxx = px && ahx != 0.0f, d_yxy = px && aiy != 0.0f, d_zxz = px && aiz != 0.0f;
+        const bool d_xxy = py && aix != 0.0f, d_yyy = py && ahy != 0.0f, d_zyz = py && aiz != 0.0f;
+        const bool d_xxz = pz && aix != 0.0f, d_yyz = pz && aiy != 0.0f, d_zzz = pz && ahz != 0.0f;
+        const float m_xxx = mem_o(F.m_dxxx, q, d_xxx), m_yxy = mem_o(F.m_dyxy, q, d_yxy);
+        const float m_zxz = mem_o(F.m_dzxz, q, d_zxz), m_xxy = mem_o(F.m_dxxy, q, d_xxy);
+        const float m_yyy = mem_o(F.m_dyyy, q, d_yyy), m_zyz = mem_o(F.m_dzyz, q, d_zyz);
+        const float m_xxz = mem_o(F.m_dxxz, q, d_xxz), m_yyz = mem_o(F.m_dyyz, q, d_yyz);
+        const float m_zzz = mem_o(F.m_dzzz, q, d_zzz);
         // x stencils of this plane from the lanes (all lanes take part)
         const float cxx = cur.cxx, cxy = cur.cxy;
         const float sx_xx = sten_lanes<R>(cxx, l, -1, c);    // d-x sxx
         const float sx_xy = sten_lanes<R>(cxy, l, 0, c);     // d+x sxy
         const float sx_xz = sten_lanes<R>(qa[R], l, 0, c);   // d+x sxz
         if (own) {
-            const int kk = k + pml - 1;
-            const bool zin = !((!fs && k <= 0) || k >= nz + 1);
             unsigned yo[2 * R + 1];  // rows j - R .. j + R of this plane
 #pragma unroll
             for (int m = 0; m <= 2 * R; ++m) yo[m] = q + unsigned(m - R) * syb;
@@ -437,11 +446,9 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
 #pragma unroll
                 for (int m = 2; m <= R; ++m) e = e + c.c[m - 1] * (qa[R + m] - qa[R - m + 1]);
                 float pdxxx = idx * sx_xx, pdyxy = idy * sten_y<R>(sxy, yo, 0, c), pdzxz = idz * e;
-                if (!Xin || !yin || !zin) {
-                    pdxxx = damp_o(F.m_dxxx, q, pdxxx, P.dhx[ii], P.ahx[ii], adt);
-                    pdyxy = damp_o(F.m_dyxy, q, pdyxy, P.diy[jj], P.aiy[jj], adt);
-                    pdzxz = damp_o(F.m_dzxz, q, pdzxz, P.diz[kk], P.aiz[kk], adt);
-                }
+                pdxxx = damp_o(F.m_dxxx, q, pdxxx, ahx, bhx, m_xxx, d_xxx);
+                pdyxy = damp_o(F.m_dyxy, q, pdyxy, aiy, biy, m_yxy, d_yxy);
+                pdzxz = damp_o(F.m_dzxz, q, pdzxz, aiz, biz, m_zxz, d_zxz);
                 sto(O.vx, q, cur.vx + dt / cur.rx * (pdxxx + pdyxy + pdzxz));
             }
             // ---- vy (i, Y, k)
@@ -450,11 +457,9 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
 #pragma unroll
                 for (int m = 2; m <= R; ++m) e = e + c.c[m - 1] * (qb[R + m] - qb[R - m + 1]);
                 float pdxxy = idx * sx_xy, pdyyy = idy * sten_y<R>(syy, yo, -1, c), pdzyz = idz * e;
-                if (!xin || !Yin || !zin) {
-                    pdxxy = damp_o(F.m_dxxy, q, pdxxy, P.dix[ii], P.aix[ii], adt);
-                    pdyyy = damp_o(F.m_dyyy, q, pdyyy, P.dhy[jj], P.ahy[jj], adt);
-                    pdzyz = damp_o(F.m_dzyz, q, pdzyz, P.diz[kk], P.aiz[kk], adt);
-                }
+                pdxxy = damp_o(F.m_dxxy, q, pdxxy, aix, bix, m_xxy, d_xxy);
+                pdyyy = damp_o(F.m_dyyy, q, pdyyy, ahy, bhy, m_yyy, d_yyy);
+                pdzyz = damp_o(F.m_dzyz, q, pdzyz, aiz, biz, m_zyz, d_zyz);
                 sto(O.vy, q, cur.vy + dt / cur.ry * (pdxxy + pdyyy + pdzyz));
             }
             // ---- vz (i, j, Z = k)
@@ -463,12 +468,9 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
 #pragma unroll
                 for (int m = 2; m <= R; ++m) e = e + c.c[m - 1] * (qc[R + m - 1] - qc[R - m]);
                 float pdxxz = idx * sx_xz, pdyyz = idy * sten_y<R>(syz, yo, 0, c), pdzzz = idz * e;
-                const bool Zin = !((!fs && k <= 1) || k >= nz + 1);
-                if (!xin || !yin || !Zin) {
-                    pdxxz = damp_o(F.m_dxxz, q, pdxxz, P.dix[ii], P.aix[ii], adt);
-                    pdyyz = damp_o(F.m_dyyz, q, pdyyz, P.diy[jj], P.aiy[jj], adt);
-                    pdzzz = damp_o(F.m_dzzz, q, pdzzz, P.dhz[kk], P.ahz[kk], adt);
-                }
+                pdxxz = damp_o(F.m_dxxz, q, pdxxz, aix, bix, m_xxz, d_xxz);
+                pdyyz = damp_o(F.m_dyyz, q, pdyyz, aiy, biy, m_yyz, d_yyz);
+                pdzzz = damp_o(F.m_dzzz, q, pdzzz, ahz, bhz, m_zzz, d_zzz);
                 sto(O.vz, q, cur.vz + dt / cur.rz * (pdxxz + pdyyz + pdzzz));
             }
         }
@@ -922,11 +924,18 @@ inline size_t model_index(const owl_elastic3d* b, const ShotHostE& H, int i, int
 // 1D CFS-MPML profile of one axis (module_cfspml.f90:498-620): for i <= 1
 // (unless the top is a free surface) and i >= n, nd = |i - edge| / pml,
 // d0 = ln(1/R0) (2 + 1) pmlvp / (2 pml d) nd^2, alpha = max(alphamax (1 -
-// nd), alphamax / 4); zero elsewhere.  Arrays di, dh, ai, ah of n + 2 pml.
-void mpml_axis(int n, int pml, float d, float pmlvp, float alphamax, bool top_off, std::vector<float>& out) {
+// nd), alphamax / 4); zero elsewhere.  From d0 and alpha the coefficients of
+// the memory variable (damp_coef, module_wavefield.f90:40-47, the same FP32
+// operations): arrays ai, ah, bi, bh of n + 2 pml.
+void mpml_axis(int n, int pml, float d, float pmlvp, float alphamax, bool top_off, float dt, std::vector<float>& out) {
     const int len = n + 2 * pml;
-    std::vector<float> di(len, 0.f), dh(len, 0.f), ai(len, 0.f), ah(len, 0.f);
-    const float R0 = 1.0e-5f, extra = 0.25f * alphamax, lg = std::log(1.0f / R0);
+    std::vector<float> ai(len, 0.f), ah(len, 0.f), bi(len, 0.f), bh(len, 0.f);
+    const float R0 = 1.0e-5f, extra = 0.25f * alphamax, lg = std::log(1.0f / R0), adt = std::fabs(dt);
+    auto coef = [&](float d0, float alpha, float& a, float& b) {
+        if (d0 == 0.0f) return;
+        a = -(2.0f * adt * d0 / (2.0f + adt * (d0 + alpha)));
+        b = (2.0f - adt * (d0 + alpha)) / (2.0f + adt * (d0 + alpha));
+    };
     for (int i = -pml + 1; i <= n + pml; ++i) {
         int side = 0;
         if (!top_off && i <= 1) side = -1;
@@ -935,12 +944,12 @@ void mpml_axis(int n, int pml, float d, float pmlvp, float alphamax, bool top_of
         const int ref = side < 0 ? 1 : n, q = i + pml - 1;
         const float nd = float(std::abs(i - ref)) * 1.0f / float(pml);
         const float ndh = std::fabs(float(i - ref) - 0.5f) * 1.0f / float(pml);
-        di[q] = lg * (2 + 1.0f) * pmlvp / (2.0f * float(pml) * d) * (nd * nd);
-        dh[q] = lg * (2 + 1.0f) * pmlvp / (2.0f * float(pml) * d) * (ndh * ndh);
-        ai[q] = std::max(alphamax * (1.0f - nd), extra);
-        ah[q] = std::max(alphamax * (1.0f - ndh), extra);
+        coef(lg * (2 + 1.0f) * pmlvp / (2.0f * float(pml) * d) * (nd * nd), std::max(alphamax * (1.0f - nd), extra),
+             ai[q], bi[q]);
+        coef(lg * (2 + 1.0f) * pmlvp / (2.0f * float(pml) * d) * (ndh * ndh), std::max(alphamax * (1.0f - ndh), extra),
+             ah[q], bh[q]);
     }
-    for (auto* v : {&di, &dh, &ai, &ah}) out.insert(out.end(), v->begin(), v->end());
+    for (auto* v : {&ai, &ah, &bi, &bh}) out.insert(out.end(), v->begin(), v->end());
 }
 
 void retile_e(owl_elastic3d* b) {
@@ -1061,9 +1070,9 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
         b->pts_full += double(H.nx + 2 * pml) * double(H.ny + 2 * pml) * double(H.nz + 2 * pml);
         S.prof = prof;
         const float amax = float(double(1.0f * f0max) * M_PI);
-        mpml_axis(H.nx, pml, cfg->dx, pmlvp, amax, false, profs);
-        mpml_axis(H.ny, pml, cfg->dy, pmlvp, amax, false, profs);
-        mpml_axis(H.nz, pml, cfg->dz, pmlvp, amax, b->fs != 0, profs);
+        mpml_axis(H.nx, pml, cfg->dx, pmlvp, amax, false, cfg->dt, profs);
+        mpml_axis(H.ny, pml, cfg->dy, pmlvp, amax, false, cfg->dt, profs);
+        mpml_axis(H.nz, pml, cfg->dz, pmlvp, amax, b->fs != 0, cfg->dt, profs);
         prof += 4 * (H.nx + 2 * pml) + 4 * (H.ny + 2 * pml) + 4 * (H.nz + 2 * pml);
         S.nr = int(H.rec.size());
         S.trace0 = trace;
