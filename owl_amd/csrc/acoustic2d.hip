@@ -23,6 +23,7 @@
 
 #include "common.hpp"
 #include "host_prep.hpp"
+#include "launch_shape.hpp"
 #include "ordered_sum.hpp"
 #include "owl_amd.h"
 
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(256) void k_step_fused(const Shot* __restrict__ sho
     // one wavefront per tile (blockDim.x = 64): the tile, its shot and every
     // row index are wavefront-uniform, so they live in scalar registers and
     // the per-row PML coefficients come through scalar loads
-    const int tile = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * int(blockDim.y) + int(threadIdx.y));
+    const int tile = __builtin_amdgcn_readfirstlane(xcd_block() * int(blockDim.y) + int(threadIdx.y));
     if (tile >= nftile) return;
     const Shot S = shots[ftile_shot[tile]];
     const int lt = tile - S.ftile0;
@@ -922,7 +923,7 @@ __global__ __launch_bounds__(256) void k_adj_fused(const Shot* __restrict__ shot
     // one wavefront per tile (blockDim.x = 64): the tile, its shot and every
     // row index are wavefront-uniform, so they live in scalar registers and
     // the per-row PML coefficients come through scalar loads
-    const int tile = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * int(blockDim.y) + int(threadIdx.y));
+    const int tile = __builtin_amdgcn_readfirstlane(xcd_block() * int(blockDim.y) + int(threadIdx.y));
     if (tile >= nftile) return;
     const Shot S = shots[ftile_shot[tile]];
     const int lt = tile - S.atile0;

@@ -109,9 +109,9 @@ __device__ __forceinline__ void sto(float* base, unsigned off, float v) {
 }
 
 // Memory-variable update m = a d + b m, d = (d + m) / kappa with kappa = 1
-// (module_wavefield.f90:60-66).
-__device__ __forceinline__ float mpml(float* m, unsigned qb, float d, float a, float b) {
-    const float v = a * d + b * ldo(m, qb);
+// (module_wavefield.f90:60-66); the old m is loaded with the row's inputs.
+__device__ __forceinline__ float mpml(float* m, unsigned qb, float d, float a, float b, float m0) {
+    const float v = a * d + b * m0;
     sto(m, qb, v);
     return d + v;
 }
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256) void k2e_stress(const ShotE2* __restrict__ sho
     constexpr int W = 64 - 2 * R;
     // one wavefront per tile (blockDim.x = 64): tile, shot and row indices
     // are wavefront-uniform and live in scalar registers
-    const int tile = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * int(blockDim.y) + int(threadIdx.y));
+    const int tile = __builtin_amdgcn_readfirstlane(xcd_block() * int(blockDim.y) + int(threadIdx.y));
     const ShotE2 S = shots[tile_shot[tile]];
     int lt = tile - S.tile0;
     const int tx = lt % S.ntx, tz = lt / S.ntx;
@@ -173,46 +173,79 @@ __global__ __launch_bounds__(256) void k2e_stress(const ShotE2* __restrict__ sho
         qz[m] = mcol ? ldo(vz, r) : 0.0f;
     }
     const bool xin = !(i <= 0 || i >= nx + 1), Xin = !(i <= 1 || i >= nx + 1);
-    for (int j = j0; j <= j1; ++j, q += szb) {
-        {
-            const unsigned r = q + unsigned(R) * szb;
-            qx[2 * R] = mcol ? ldo(vx, r) : 0.0f;
-            qz[2 * R] = mcol ? ldo(vz, r) : 0.0f;
+    const float axi = own ? P.axi[ii] : 0.0f, bxi = own ? P.bxi[ii] : 0.0f;
+    const float axh = own ? P.axh[ii] : 0.0f, bxh = own ? P.bxh[ii] : 0.0f;
+    // The inputs of one row: the queues' fronts (row j + R) and, on the owned
+    // lanes, the moduli, the old stresses and the memory variables the row
+    // damps (dn at the nodes, dz also along z there, ds at the corners).
+    // Row j + 1's are loaded while row j is computed; loaded where they were
+    // used, each group waited for its own round trip to memory.
+    struct Row {
+        float fx, fz, c11, c13, mu, sxx, szz, sxz, mxx, mzz, mxz, mzx;
+        bool dn, dz, ds;
+    };
+    auto load = [&](int j, unsigned qr, Row& w) {
+        const unsigned r = qr + unsigned(R) * szb;
+        w.dn = own && (!xin || (!FS && j <= 0) || j >= nz + 1);
+        w.dz = w.dn && !(FS && j == 1);
+        w.ds = own && (!FS || j >= 2) && (!Xin || (!FS && j <= 1) || j >= nz + 1);
+        w.fx = mcol ? ldo(vx, r) : 0.0f;
+        w.fz = mcol ? ldo(vz, r) : 0.0f;
+        if (own) {
+            w.c11 = ldo(M.c11, qr);
+            w.c13 = ldo(M.c13, qr);
+            w.mu = ldo(M.mu, qr);
+            w.sxx = ldo(F.sxx, qr);
+            w.szz = ldo(F.szz, qr);
+            w.sxz = ldo(F.sxz, qr);
         }
+        if (w.dn) w.mxx = ldo(F.m_dxvx, qr);
+        if (w.dz) w.mzz = ldo(F.m_dzvz, qr);
+        if (w.ds) {
+            w.mxz = ldo(F.m_dxvz, qr);
+            w.mzx = ldo(F.m_dzvx, qr);
+        }
+    };
+    Row cur{}, nxt{};
+    load(j0, q, cur);
+    for (int j = j0; j <= j1; ++j, q += szb) {
+        if (j < j1) load(j + 1, q + szb, nxt);
+        qx[2 * R] = cur.fx;
+        qz[2 * R] = cur.fz;
         const float sxvx = sten_lanes<R>(qx[R], l, 0, c.c);   // d+x vx
         const float sxvz = sten_lanes<R>(qz[R], l, -1, c.c);  // d-x vz
         if (own) {
             const int jj = j + pml - 1;
             {
-                const float c11 = ldo(M.c11, q), c13 = ldo(M.c13, q);
+                const float c11 = cur.c11, c13 = cur.c13;
                 float pdxvx = idx * sxvx, pdzvz;
                 if (FS && j == 1) {
                     // the surface row: dz vz from the traction condition, x damping only
-                    if (!xin) pdxvx = mpml(F.m_dxvx, q, pdxvx, P.axi[ii], P.bxi[ii]);
+                    if (cur.dn) pdxvx = mpml(F.m_dxvx, q, pdxvx, axi, bxi, cur.mxx);
                     pdzvz = -(c13 / c11 * pdxvx);
                 } else {
                     float b = c.c[0] * (qz[R + 1] - qz[R]);
 #pragma unroll
                     for (int m = 2; m <= R; ++m) b = b + c.c[m - 1] * (qz[R + m] - qz[R - m + 1]);
                     pdzvz = FS ? idz * b * sci[j] : idz * b;
-                    if (!xin || (!FS && j <= 0) || j >= nz + 1) {
-                        pdxvx = mpml(F.m_dxvx, q, pdxvx, P.axi[ii], P.bxi[ii]);
-                        pdzvz = mpml(F.m_dzvz, q, pdzvz, P.azi[jj], P.bzi[jj]);
+                    if (cur.dn) {
+                        pdxvx = mpml(F.m_dxvx, q, pdxvx, axi, bxi, cur.mxx);
+                        pdzvz = mpml(F.m_dzvz, q, pdzvz, P.azi[jj], P.bzi[jj], cur.mzz);
                     }
                 }
-                sto(O.sxx, q, ldo(F.sxx, q) + dt * (c11 * pdxvx + c13 * pdzvz));
-                sto(O.szz, q, ldo(F.szz, q) + dt * (c13 * pdxvx + c11 * pdzvz));
+                sto(O.sxx, q, cur.sxx + dt * (c11 * pdxvx + c13 * pdzvz));
+                sto(O.szz, q, cur.szz + dt * (c13 * pdxvx + c11 * pdzvz));
             }
             if (!FS || j >= 2) {
                 float a = c.c[0] * (qx[R] - qx[R - 1]);        // d-z vx
 #pragma unroll
                 for (int m = 2; m <= R; ++m) a = a + c.c[m - 1] * (qx[R + m - 1] - qx[R - m]);
                 float pdzvx = FS ? idz * a * sch[j] : idz * a, pdxvz = idx * sxvz;
-                if (!Xin || (!FS && j <= 1) || j >= nz + 1) {
-                    pdxvz = mpml(F.m_dxvz, q, pdxvz, P.axh[ii], P.bxh[ii]);
-                    pdzvx = mpml(F.m_dzvx, q, pdzvx, P.azh[jj], P.bzh[jj]);
+                if (cur.ds) {
+                    pdxvz = mpml(F.m_dxvz, q, pdxvz, axh, bxh, cur.mxz);
+                    pdzvx = mpml(F.m_dzvx, q, pdzvx, P.azh[jj], P.bzh[jj], cur.mzx);
                 }
-                sto(O.sxz, q, ldo(F.sxz, q) + dt * ldo(M.mu, q) * (pdzvx + pdxvz));
+                sto(O.sxz, q, cur.sxz + dt * cur.mu * (pdzvx + pdxvz));
             }
         }
 #pragma unroll
@@ -220,6 +253,7 @@ __global__ __launch_bounds__(256) void k2e_stress(const ShotE2* __restrict__ sho
             qx[m] = qx[m + 1];
             qz[m] = qz[m + 1];
         }
+        cur = nxt;
     }
 }
 
@@ -236,7 +270,7 @@ __global__ __launch_bounds__(256) void k2e_velocity(const ShotE2* __restrict__ s
     constexpr int W = 64 - 2 * R;
     // one wavefront per tile (blockDim.x = 64): tile, shot and row indices
     // are wavefront-uniform and live in scalar registers
-    const int tile = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * int(blockDim.y) + int(threadIdx.y));
+    const int tile = __builtin_amdgcn_readfirstlane(xcd_block() * int(blockDim.y) + int(threadIdx.y));
     const ShotE2 S = shots[tile_shot[tile]];
     int lt = tile - S.tile0;
     const int tx = lt % S.ntx, tz = lt / S.ntx;
@@ -264,13 +298,44 @@ __global__ __launch_bounds__(256) void k2e_velocity(const ShotE2* __restrict__ s
         qc[m] = mcol ? ldo(szz, r) : 0.0f;
     }
     const bool xin = !(i <= 0 || i >= nx + 1), Xin = !(i <= 1 || i >= nx + 1);
-    for (int j = j0; j <= j1; ++j, q += szb) {
-        {
-            const unsigned r = q + unsigned(R) * szb;
-            qa[2 * R] = mcol ? ldo(sxz, r) : 0.0f;
-            qc[2 * R] = mcol ? ldo(szz, r) : 0.0f;
+    const float axi = own ? P.axi[ii] : 0.0f, bxi = own ? P.bxi[ii] : 0.0f;
+    const float axh = own ? P.axh[ii] : 0.0f, bxh = own ? P.bxh[ii] : 0.0f;
+    // The inputs of one row, as in the stress sweep: the queues' fronts, sxx
+    // and, on the owned lanes, the densities, the old velocities and the
+    // memory variables the row damps (dx with vx, dz with vz).
+    struct Row {
+        float fa, fc, cxx, rx, rz, vx, vz, mxx, mxz, mzx, mzz;
+        bool dx, dz;
+    };
+    auto load = [&](int j, unsigned qr, Row& w) {
+        const unsigned r = qr + unsigned(R) * szb;
+        w.dx = own && (!Xin || (!FS && j <= 0) || j >= nz + 1);
+        w.dz = own && (!FS || j >= 2) && (!xin || (!FS && j <= 1) || j >= nz + 1);
+        w.fa = mcol ? ldo(sxz, r) : 0.0f;
+        w.fc = mcol ? ldo(szz, r) : 0.0f;
+        w.cxx = mcol ? ldo(sxx, qr) : 0.0f;
+        if (own) {
+            w.rx = ldo(M.rx, qr);
+            w.rz = ldo(M.rz, qr);
+            w.vx = ldo(F.vx, qr);
+            w.vz = ldo(F.vz, qr);
         }
-        const float cxx = mcol ? ldo(sxx, q) : 0.0f;
+        if (w.dx) {
+            w.mxx = ldo(F.m_dxxx, qr);
+            w.mxz = ldo(F.m_dzxz, qr);
+        }
+        if (w.dz) {
+            w.mzx = ldo(F.m_dxxz, qr);
+            w.mzz = ldo(F.m_dzzz, qr);
+        }
+    };
+    Row cur{}, nxt{};
+    load(j0, q, cur);
+    for (int j = j0; j <= j1; ++j, q += szb) {
+        if (j < j1) load(j + 1, q + szb, nxt);
+        qa[2 * R] = cur.fa;
+        qc[2 * R] = cur.fc;
+        const float cxx = cur.cxx;
         const float sxxx = sten_lanes<R>(cxx, l, -1, c.c);    // d-x sxx
         const float sxxz = sten_lanes<R>(qa[R], l, 0, c.c);   // d+x sxz
         if (own) {
@@ -280,22 +345,22 @@ __global__ __launch_bounds__(256) void k2e_velocity(const ShotE2* __restrict__ s
 #pragma unroll
                 for (int m = 2; m <= R; ++m) b = b + c.c[m - 1] * (qa[R + m] - qa[R - m + 1]);
                 float pdxxx = idx * sxxx, pdzxz = FS ? idz * b * sci[j] : idz * b;
-                if (!Xin || (!FS && j <= 0) || j >= nz + 1) {
-                    pdxxx = mpml(F.m_dxxx, q, pdxxx, P.axh[ii], P.bxh[ii]);
-                    pdzxz = mpml(F.m_dzxz, q, pdzxz, P.azi[jj], P.bzi[jj]);
+                if (cur.dx) {
+                    pdxxx = mpml(F.m_dxxx, q, pdxxx, axh, bxh, cur.mxx);
+                    pdzxz = mpml(F.m_dzxz, q, pdzxz, P.azi[jj], P.bzi[jj], cur.mxz);
                 }
-                sto(O.vx, q, ldo(F.vx, q) + dt / ldo(M.rx, q) * (pdxxx + pdzxz));
+                sto(O.vx, q, cur.vx + dt / cur.rx * (pdxxx + pdzxz));
             }
             if (!FS || j >= 2) {
                 float b = c.c[0] * (qc[R] - qc[R - 1]);       // d-z szz
 #pragma unroll
                 for (int m = 2; m <= R; ++m) b = b + c.c[m - 1] * (qc[R + m - 1] - qc[R - m]);
                 float pdxxz = idx * sxxz, pdzzz = FS ? idz * b * sch[j] : idz * b;
-                if (!xin || (!FS && j <= 1) || j >= nz + 1) {
-                    pdxxz = mpml(F.m_dxxz, q, pdxxz, P.axi[ii], P.bxi[ii]);
-                    pdzzz = mpml(F.m_dzzz, q, pdzzz, P.azh[jj], P.bzh[jj]);
+                if (cur.dz) {
+                    pdxxz = mpml(F.m_dxxz, q, pdxxz, axi, bxi, cur.mzx);
+                    pdzzz = mpml(F.m_dzzz, q, pdzzz, P.azh[jj], P.bzh[jj], cur.mzz);
                 }
-                sto(O.vz, q, ldo(F.vz, q) + dt / ldo(M.rz, q) * (pdxxz + pdzzz));
+                sto(O.vz, q, cur.vz + dt / cur.rz * (pdxxz + pdzzz));
             }
         }
 #pragma unroll
@@ -303,6 +368,7 @@ __global__ __launch_bounds__(256) void k2e_velocity(const ShotE2* __restrict__ s
             qa[m] = qa[m + 1];
             qc[m] = qc[m + 1];
         }
+        cur = nxt;
     }
 }
 
