@@ -32,7 +32,6 @@ namespace a2 {
 
 constexpr int kBX = 64;     // threads along x (one wavefront per row)
 constexpr int kBY = 4;      // rows of threads per block
-constexpr int kRows = 16;   // z rows per block (kRows / kBY per thread)
 constexpr int kPitchAlign = 64;  // row pitch multiple, floats (256 B)
 
 struct Coef {
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_p(const Shot* __restrict__
                                                         const float* __restrict__ bk,
                                                         const float* __restrict__ prof, Coef c,
                                                         float dt, float idx, float idz, int pml,
-                                                        int free_surface) {
+                                                        int free_surface, int rpt) {
     const int tile = blockIdx.x;
     const Shot S = shots[shot_of_tile(tile_shot, tile)];
     const FieldSet F = sets.s[blockIdx.y];
@@ -119,10 +118,9 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_p(const Shot* __restrict__
         bx = bxi[i + pml - 1];
     }
     const size_t pitch = size_t(S.pitch);
-#pragma unroll
-    for (int k = 0; k < kRows / kBY; ++k) {
+    for (int k = 0; k < rpt; ++k) {
         // kBX = 64: the row is wavefront-uniform (scalar registers)
-        const int j = -pml + 1 + tz * kRows + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
+        const int j = -pml + 1 + tz * (kBY * rpt) + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
         if (j > nz + pml) break;
         if (free_surface && j < 2) continue;
         const size_t q = size_t(S.off) + size_t(i - lo) + size_t(j - lo) * pitch;
@@ -146,23 +144,10 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_p(const Shot* __restrict__
             F.m_out[1][q] = mem;
             pdz = pdz + mem;
         }
-        F.p_out[q] = F.p_in[q] - dt * bk[mq(S, q)] * (pdx + pdz);
-    }
-}
-
-// Free-surface mirror p(i, j) = -p(i, 2 - j), j <= 0 (module_wavefield.f90:145-151).
-template <int R>
-__global__ void k_mirror_p(const Shot* __restrict__ shots, Sets sets, int pml) {
-    const Shot S = shots[blockIdx.y];
-    float* p = sets.s[blockIdx.z].p_out;
-    const int lo = 1 - pml - R;
-    const int lx = S.nx + 2 * pml;
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < lx * pml; e += gridDim.x * blockDim.x) {
-        const int i = -pml + 1 + e % lx;
-        const int j = -pml + 1 + e / lx;  // j in [-pml+1, 0]
-        const size_t pitch = size_t(S.pitch);
-        p[size_t(S.off) + size_t(i - lo) + size_t(j - lo) * pitch] =
-            -p[size_t(S.off) + size_t(i - lo) + size_t(2 - j - lo) * pitch];
+        const float pn = F.p_in[q] - dt * bk[mq(S, q)] * (pdx + pdz);
+        F.p_out[q] = pn;
+        // free surface: p(i, 2 - j) = -p(i, j) (module_wavefield.f90:145-151)
+        if (free_surface && j <= pml + 1) F.p_out[q - size_t(2 * j - 2) * pitch] = -pn;
     }
 }
 
@@ -177,7 +162,7 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_v(const Shot* __restrict__
                                                         const float* __restrict__ rho,
                                                         const float* __restrict__ prof, Coef c,
                                                         float dt, float idx, float idz, int pml,
-                                                        int free_surface) {
+                                                        int free_surface, int rpt) {
     const int tile = blockIdx.x;
     const Shot S = shots[shot_of_tile(tile_shot, tile)];
     const FieldSet F = sets.s[blockIdx.y];
@@ -200,10 +185,9 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_v(const Shot* __restrict__
         bx = bxh[i + pml - 1];
     }
     const size_t pitch = size_t(S.pitch);
-#pragma unroll
-    for (int k = 0; k < kRows / kBY; ++k) {
+    for (int k = 0; k < rpt; ++k) {
         // kBX = 64: the row is wavefront-uniform (scalar registers)
-        const int j = -pml + 1 + tz * kRows + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
+        const int j = -pml + 1 + tz * (kBY * rpt) + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
         if (j > nz + pml) break;
         const size_t q = size_t(S.off) + size_t(i - lo) + size_t(j - lo) * pitch;
         if (!free_surface || j >= 1) {
@@ -781,7 +765,7 @@ __global__ __launch_bounds__(kBX * kBY) void k_adj_p(const Shot* __restrict__ sh
                                                      const int* __restrict__ tile_shot, AdjSet A,
                                                      const float* __restrict__ bk,
                                                      const float* __restrict__ prof, Coef c, float dt,
-                                                     float idx, float idz, int pml,
+                                                     float idx, float idz, int pml, int rpt,
                                                      const float* __restrict__ p_cur,
                                                      const float* __restrict__ p_prev) {
     const int tile = blockIdx.x;
@@ -799,10 +783,9 @@ __global__ __launch_bounds__(kBX * kBY) void k_adj_p(const Shot* __restrict__ sh
     const float* bzi = azi + lz;
     const bool xslab = (i <= 0 || i >= nx + 1);
     const size_t pitch = size_t(S.pitch);
-#pragma unroll
-    for (int k = 0; k < kRows / kBY; ++k) {
+    for (int k = 0; k < rpt; ++k) {
         // kBX = 64: the row is wavefront-uniform (scalar registers)
-        const int j = -pml + 1 + tz * kRows + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
+        const int j = -pml + 1 + tz * (kBY * rpt) + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
         if (j > nz + pml) break;
         const size_t q = size_t(S.off) + size_t(i - lo) + size_t(j - lo) * pitch;
         float sx = 0.0f, sz = 0.0f;
@@ -837,7 +820,7 @@ __global__ __launch_bounds__(kBX * kBY) void k_adj_v(const Shot* __restrict__ sh
                                                      const int* __restrict__ tile_shot, AdjSet A,
                                                      const float* __restrict__ rho,
                                                      const float* __restrict__ prof, Coef c, float dt,
-                                                     float idx, float idz, int pml,
+                                                     float idx, float idz, int pml, int rpt,
                                                      const float* __restrict__ vx_cur,
                                                      const float* __restrict__ vx_prev,
                                                      const float* __restrict__ vz_cur,
@@ -857,10 +840,9 @@ __global__ __launch_bounds__(kBX * kBY) void k_adj_v(const Shot* __restrict__ sh
     const float* bzh = azh + lz;
     const bool xslab = (i <= 1 || i >= nx + 1);
     const size_t pitch = size_t(S.pitch);
-#pragma unroll
-    for (int k = 0; k < kRows / kBY; ++k) {
+    for (int k = 0; k < rpt; ++k) {
         // kBX = 64: the row is wavefront-uniform (scalar registers)
-        const int j = -pml + 1 + tz * kRows + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
+        const int j = -pml + 1 + tz * (kBY * rpt) + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
         if (j > nz + pml) break;
         const size_t q = size_t(S.off) + size_t(i - lo) + size_t(j - lo) * pitch;
         const float rx = 0.5f * (rho[mq(S, q)] + rho[mq(S, q) - 1]);
@@ -1350,6 +1332,7 @@ struct owl_acoustic2d {
     std::vector<ShotHost> hs;
     std::vector<Shot> sd;          // device descriptors (host copy)
     std::vector<int> tile_shot;
+    int rpt = 1;                   // rows a thread of the sweeps updates (sweep_tiling)
     size_t field_elems = 0;        // elements of one field buffer (all shots)
     size_t model_elems = 0;        // elements of bk / rho (one padded grid per distinct window)
     size_t grad_elems = 0;         // sum of nx*nz
@@ -1508,6 +1491,28 @@ void upload_model(owl_acoustic2d* b) {
     OWL_HIP(hipStreamSynchronize(b->stream));
 }
 
+// Tiles of the sweeps: 64 columns and kBY rpt rows.  A thread updates its rpt
+// rows one after another (the stores keep the next row's loads behind them),
+// so a small batch gives every row a thread of its own and a large one,
+// which fills the chip anyway, reads its block's tables once for 4 rows.  us
+// per forward step at 1 / 2 / 4 rows: 461 x 461 nodes, 1 shot 13.4 / 15.6 /
+// 20.4, 2 shots 16.2 / 17.9 / 22.7, 4 shots 23.0 / 21.8 / 26.0, 8 shots 35.9
+// / 33.5 / 32.2, 16 shots 57.0 / 53.5 / 51.9.
+void sweep_tiling(owl_acoustic2d* b) {
+    b->tile_shot.clear();
+    double waves = 0;  // wavefronts at one row each
+    for (const Shot& S : b->sd)
+        waves += double((S.nx + 2 * b->pml + kBX - 1) / kBX) * double(S.nz + 2 * b->pml);
+    b->rpt = waves < 10000 ? 1 : (waves < 20000 ? 2 : 4);
+    for (size_t s = 0; s < b->sd.size(); ++s) {
+        Shot& S = b->sd[s];
+        S.tile0 = int(b->tile_shot.size());
+        S.ntx = (S.nx + 2 * b->pml + kBX - 1) / kBX;
+        const int ntz = (S.nz + 2 * b->pml + kBY * b->rpt - 1) / (kBY * b->rpt);
+        b->tile_shot.insert(b->tile_shot.end(), size_t(S.ntx) * ntz, int(s));
+    }
+}
+
 // Column-strip tiles of the fused step: 64 - (2R - 1) output columns and
 // fzc rows each, one wavefront per tile.
 void fused_tiling(owl_acoustic2d* b) {
@@ -1568,7 +1573,6 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
 
     b->hs.assign(nshot, ShotHost{});
     b->sd.assign(nshot, Shot{});
-    b->tile_shot.clear();
     long long off = 0, moff = 0, strip = 0, trace = 0, g0 = 0;
     int edge = 0, prof = 0;
     std::vector<float> profs, amp;
@@ -1652,10 +1656,6 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
             }
             S.mdel = mo - S.off;
         }
-        S.tile0 = int(b->tile_shot.size());
-        S.ntx = (H.nx + 2 * pml + kBX - 1) / kBX;
-        const int ntz = (H.nz + 2 * pml + kRows - 1) / kRows;
-        b->tile_shot.insert(b->tile_shot.end(), size_t(S.ntx) * ntz, s);
         b->pts_full += double(H.nx + 2 * pml) * double(H.nz + 2 * pml);
         S.prof = prof;
         PmlAxis px = cfspml_axis(H.nx, pml, cfg->dx, cfg->dt, pmlvp, H.f0max);
@@ -1861,6 +1861,7 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
         OWL_HIP(hipEventCreate(&b->ev1));
     }
     hipStream_t st = b->stream;
+    sweep_tiling(b);
     fused_tiling(b);
     b->d_shots.upload(b->sd, st);
     b->d_tile_shot.upload(b->tile_shot, st);
@@ -1981,15 +1982,11 @@ void launch_step(owl_acoustic2d* b, const Sets& sets, int nsets, float dt) {
     const StepBytes sb = b->profiling ? step_bytes(b, nsets) : StepBytes{0, 0};
     int ev = prof_begin(b, nsets == 2 ? kKP2 : kKP, sb.p);
     hipLaunchKernelGGL(k_update_p<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), sets,
-                       b->d_bk.get(), b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs);
+                       b->d_bk.get(), b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs, b->rpt);
     prof_end(b, ev);
-    if (fs) {
-        const dim3 g2(64, unsigned(b->sd.size()), unsigned(nsets));
-        hipLaunchKernelGGL(k_mirror_p<R>, g2, dim3(256), 0, b->stream, b->d_shots.get(), sets, b->pml);
-    }
     ev = prof_begin(b, nsets == 2 ? kKV2 : kKV, sb.v);
     hipLaunchKernelGGL(k_update_v<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), sets,
-                       b->d_rho.get(), b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs);
+                       b->d_rho.get(), b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs, b->rpt);
     prof_end(b, ev);
 }
 
@@ -2404,13 +2401,13 @@ void adjoint_step(owl_acoustic2d* b, int t, const float* const* cur, const float
     // p-pass: ex, ez, ph, bk, p_t, p_{t-1}, psx/psz read; ph, dx, dz written; gK r+w
     int ev = prof_begin(b, 10, pts * (5 * 4 + 3 * 4 + 16) + 4.0 * b->pts_model);
     hipLaunchKernelGGL(k_adj_p<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), A, b->d_bk.get(),
-                       b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, cur[0], prev[0]);
+                       b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, b->rpt, cur[0], prev[0]);
     prof_end(b, ev);
     src_correction(b, t);
     // v-pass: dx, dz, vxh, vzh, rho, 4 states read; vxh, vzh, ex, ez written; gX, gZ r+w
     ev = prof_begin(b, 11, pts * (8 * 4 + 4 * 4 + 32) + 4.0 * b->pts_model);
     hipLaunchKernelGGL(k_adj_v<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), A, b->d_rho.get(),
-                       b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, cur[1], prev[1], cur[2], prev[2]);
+                       b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, b->rpt, cur[1], prev[1], cur[2], prev[2]);
     prof_end(b, ev);
     inject_residual(b, t);
 }
