@@ -136,6 +136,11 @@ __device__ __forceinline__ float sten_lanes(float v, int l, int off, const float
 // over rows j-R .. j+R of vx and vz; x stencils from the other lanes' current
 // rows by shuffles, so a wavefront of 64 lanes updates the middle 64 - 2R
 // columns and the others only feed them.
+// Free surface (module_wavefield.f90:223-245): szz(1) = 0 and the odd stress
+// mirrors szz(1-j) = -szz(1+j), sxx(1-j) = -sxx(1+j), sxz(2-j) = -sxz(1+j),
+// j = 1 .. R, written with the rows they mirror.  The velocities above the
+// surface stay zero throughout (no sweep, source or record writes them),
+// which is what OWL's update zeroes them to.
 // ---------------------------------------------------------------------------
 template <int R, bool FS>
 __global__ __launch_bounds__(256) void k2e_stress(const ShotE2* __restrict__ shots, const int* __restrict__ tile_shot,
@@ -233,8 +238,15 @@ __global__ __launch_bounds__(256) void k2e_stress(const ShotE2* __restrict__ sho
                         pdzvz = mpml(F.m_dzvz, q, pdzvz, P.azi[jj], P.bzi[jj], cur.mzz);
                     }
                 }
-                sto(O.sxx, q, cur.sxx + dt * (c11 * pdxvx + c13 * pdzvz));
-                sto(O.szz, q, cur.szz + dt * (c13 * pdxvx + c11 * pdzvz));
+                const float nxx = cur.sxx + dt * (c11 * pdxvx + c13 * pdzvz);
+                const float nzz = FS && j == 1 ? 0.0f : cur.szz + dt * (c13 * pdxvx + c11 * pdzvz);
+                sto(O.sxx, q, nxx);
+                sto(O.szz, q, nzz);
+                if (FS && j >= 2 && j <= R + 1) {  // odd mirrors: row 2 - j
+                    const unsigned qm = q - unsigned(2 * j - 2) * szb;
+                    sto(O.sxx, qm, -nxx);
+                    sto(O.szz, qm, -nzz);
+                }
             }
             if (!FS || j >= 2) {
                 float a = c.c[0] * (qx[R] - qx[R - 1]);        // d-z vx
@@ -245,7 +257,9 @@ __global__ __launch_bounds__(256) void k2e_stress(const ShotE2* __restrict__ sho
                     pdxvz = mpml(F.m_dxvz, q, pdxvz, axh, bxh, cur.mxz);
                     pdzvx = mpml(F.m_dzvx, q, pdzvx, P.azh[jj], P.bzh[jj], cur.mzx);
                 }
-                sto(O.sxz, q, cur.sxz + dt * cur.mu * (pdzvx + pdxvz));
+                const float nxz = cur.sxz + dt * cur.mu * (pdzvx + pdxvz);
+                sto(O.sxz, q, nxz);
+                if (FS && j <= R + 1) sto(O.sxz, q - unsigned(2 * j - 3) * szb, -nxz);  // row 3 - j
             }
         }
 #pragma unroll
@@ -369,24 +383,6 @@ __global__ __launch_bounds__(256) void k2e_velocity(const ShotE2* __restrict__ s
             qc[m] = qc[m + 1];
         }
         cur = nxt;
-    }
-}
-
-// Free surface, after the stress sweep (module_wavefield.f90:223-245): the
-// odd stress mirrors szz(1-j) = -szz(1+j), sxx(1-j) = -sxx(1+j),
-// sxz(2-j) = -sxz(1+j), j = 1 .. R, and szz(1) = 0, over every stored
-// column.  The velocities above the surface stay zero throughout (no sweep,
-// source or record writes them), which is what OWL's update zeroes them to.
-__global__ void k2e_fs_mirror(const ShotE2* __restrict__ shots, float* sxx, float* szz, float* sxz, int pml, int R) {
-    const ShotE2 S = shots[blockIdx.y];
-    const int lo = 1 - pml - R, w = S.nx + 2 * (pml + R);
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < w * R; e += gridDim.x * blockDim.x) {
-        const int i = lo + e % w, j = 1 + e / w;
-        const size_t up = at2(S, lo, i, 1 + j);
-        szz[at2(S, lo, i, 1 - j)] = -szz[up];
-        sxx[at2(S, lo, i, 1 - j)] = -sxx[up];
-        sxz[at2(S, lo, i, 2 - j)] = -sxz[up];
-        if (j == 1) szz[at2(S, lo, i, 1)] = 0.0f;
     }
 }
 
@@ -1209,14 +1205,6 @@ void step2(owl_elastic2d* b, const EF2& F, const EV2& O, float dt, double bs, do
         hipLaunchKernelGGL((k2e_stress<R, false>), grd, blk, 0, st, b->d_shots.get(), b->d_tile_shot.get(), F, O, M,
                            b->d_prof.get(), b->d_sc.get(), b->coef, dt, b->idx, b->idz, b->pml, b->kc);
     b->prof.end(st, ev);
-    if (b->fs) {
-        ev = b->prof.begin(st, 5, 0);
-        int w = 1;
-        for (auto& S : b->sd) w = std::max(w, (S.nx + 2 * (b->pml + b->R)) * b->R);
-        hipLaunchKernelGGL(k2e_fs_mirror, dim3(unsigned((w + 255) / 256), unsigned(b->sd.size())), dim3(256), 0, st,
-                           b->d_shots.get(), O.sxx, O.szz, O.sxz, b->pml, b->R);
-        b->prof.end(st, ev);
-    }
     ev = b->prof.begin(st, 1, bv);
     if (b->fs)
         hipLaunchKernelGGL((k2e_velocity<R, true>), grd, blk, 0, st, b->d_shots.get(), b->d_tile_shot.get(), F, O,

@@ -87,6 +87,7 @@ struct Tap {
 // which may lie outside the grid where those weights are 0.
 struct RecBox {
     long long cell0;
+    int kz0;  // plane of the box's first cells
     float w[3][2 * kNkw + 1];
 };
 
@@ -165,6 +166,14 @@ __device__ __forceinline__ Prof prof_of(const float* prof, const ShotE& S, int p
 // (X, j, Z), sxy at (X, Y, k), all stored at the same index (i, j, k).
 // module_wavefield.f90:58-306 (free surface :592-821).  The z stencils come
 // from register queues over planes k-R .. k+R of vx, vy, vz.
+// Free surface (module_wavefield.f90:823-845): szz(1) = 0 and the odd stress
+// mirrors about plane 1 (sxx, syy, szz, sxy onto plane 2-k, syz, sxz onto
+// 3-k, k = 2 .. R+1), written with the planes they mirror.  The velocities
+// above the surface stay zero throughout (no sweep, source or record writes
+// them), which is what OWL's update zeroes them to (:580-590); the
+// receivers read them mirrored (ke_record).  As launches of their own over
+// whole planes these four steps took 45 us of a 4.0 ms step of 8 shots and
+// a tenth of one of 2 small shots.
 // ---------------------------------------------------------------------------
 template <int R>
 __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots, const int* __restrict__ tile_shot,
@@ -289,9 +298,18 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
                     for (int m = 2; m <= R; ++m) s = s + c.c[m - 1] * (qz[R + m] - qz[R - m + 1]);
                     pdzvz = damp_o(F.m_dzvz, q, idz * s, aiz, biz, m_zvz, d_zvz);
                 }
-                sto(O.sxx, q, cur.sxx + dt * (c11 * pdxvx + c12 * pdyvy + c12 * pdzvz));
-                sto(O.syy, q, cur.syy + dt * (c12 * pdxvx + c11 * pdyvy + c12 * pdzvz));
-                sto(O.szz, q, cur.szz + dt * (c12 * pdxvx + c12 * pdyvy + c11 * pdzvz));
+                const float nxx = cur.sxx + dt * (c11 * pdxvx + c12 * pdyvy + c12 * pdzvz);
+                const float nyy = cur.syy + dt * (c12 * pdxvx + c11 * pdyvy + c12 * pdzvz);
+                const float nzz = top ? 0.0f : cur.szz + dt * (c12 * pdxvx + c12 * pdyvy + c11 * pdzvz);
+                sto(O.sxx, q, nxx);
+                sto(O.syy, q, nyy);
+                sto(O.szz, q, nzz);
+                if (fs && k >= 2 && k <= R + 1) {  // odd mirrors: plane 2 - k
+                    const unsigned qm = q - unsigned(2 * k - 2) * szb;
+                    sto(O.sxx, qm, -nxx);
+                    sto(O.syy, qm, -nyy);
+                    sto(O.szz, qm, -nzz);
+                }
             }
             // ---- shear stresses with a z derivative: syz, sxz (Z = k)
             if (!top) {
@@ -305,17 +323,26 @@ __global__ __launch_bounds__(256) void ke_stress(const ShotE* __restrict__ shots
                 float pdzvy = idz * a, pdyvz = idy * sten_y<R>(vz, yo, -1, c), pdzvx = idz * e, pdxvz = idx * sx_vz;
                 pdyvz = damp_o(F.m_dyvz, q, pdyvz, ahy, bhy, m_yvz, d_yvz);
                 pdzvy = damp_o(F.m_dzvy, q, pdzvy, ahz, bhz, m_zvy, d_zvy);
-                sto(O.syz, q, cur.syz + dt * cur.myz * (pdzvy + pdyvz));
+                const float nyz = cur.syz + dt * cur.myz * (pdzvy + pdyvz);
+                sto(O.syz, q, nyz);
                 pdxvz = damp_o(F.m_dxvz, q, pdxvz, ahx, bhx, m_xvz, d_xvz);
                 pdzvx = damp_o(F.m_dzvx, q, pdzvx, ahz, bhz, m_zvx, d_zvx);
-                sto(O.sxz, q, cur.sxz + dt * cur.mxz * (pdzvx + pdxvz));
+                const float nxz = cur.sxz + dt * cur.mxz * (pdzvx + pdxvz);
+                sto(O.sxz, q, nxz);
+                if (fs && k <= R + 1) {  // plane 3 - k
+                    const unsigned qm = q - unsigned(2 * k - 3) * szb;
+                    sto(O.syz, qm, -nyz);
+                    sto(O.sxz, qm, -nxz);
+                }
             }
             // ---- sxy (X, Y, k)
             {
                 float pdyvx = idy * sten_y<R>(vx, yo, -1, c), pdxvy = idx * sx_vy;
                 pdxvy = damp_o(F.m_dxvy, q, pdxvy, ahx, bhx, m_xvy, d_xvy);
                 pdyvx = damp_o(F.m_dyvx, q, pdyvx, ahy, bhy, m_yvx, d_yvx);
-                sto(O.sxy, q, cur.sxy + dt * cur.mxy * (pdyvx + pdxvy));
+                const float nxy = cur.sxy + dt * cur.mxy * (pdyvx + pdxvy);
+                sto(O.sxy, q, nxy);
+                if (fs && k >= 2 && k <= R + 1) sto(O.sxy, q - unsigned(2 * k - 2) * szb, -nxy);
             }
         }
 #pragma unroll
@@ -484,46 +511,6 @@ __global__ __launch_bounds__(256) void ke_velocity(const ShotE* __restrict__ sho
     }
 }
 
-// Free surface, whole padded x-y planes (module_wavefield.f90:580-590,
-// 823-845; submodule_forward_modeling.f90:64-73).  mode 0: zero the
-// velocities above the surface; 1: mirror the stresses; 2: mirror the
-// velocities for the receivers (NKW planes); 3: zero the velocities above
-// it over the planes modes 0 and 2 touch.
-template <int R>
-__global__ void ke_surface(const ShotE* __restrict__ shots, EF F, int pml, int mode) {
-    const ShotE S = shots[blockIdx.y];
-    const int lo = 1 - pml - R;
-    const long long plane = (long long)S.px * S.nyp;
-    const int nk = mode == 2 ? kNkw : (mode == 3 ? (R > kNkw ? R : kNkw) : R);
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < plane; e += (long long)gridDim.x * blockDim.x) {
-        const size_t b = size_t(S.off) + size_t(e);
-        auto at = [&](int k) { return b + size_t(k - lo) * size_t(S.pxy); };
-        if (mode == 0 || mode == 3) {
-            for (int m = 1; m <= nk; ++m) {
-                F.vx[at(1 - m)] = 0.0f;
-                F.vy[at(1 - m)] = 0.0f;
-                F.vz[at(2 - m)] = 0.0f;
-            }
-        } else if (mode == 1) {
-            for (int m = 1; m <= R; ++m) {
-                F.szz[at(1 - m)] = -F.szz[at(1 + m)];
-                F.szz[at(1)] = 0.0f;
-                F.sxx[at(1 - m)] = -F.sxx[at(1 + m)];
-                F.syy[at(1 - m)] = -F.syy[at(1 + m)];
-                F.sxy[at(1 - m)] = -F.sxy[at(1 + m)];
-                F.syz[at(2 - m)] = -F.syz[at(1 + m)];
-                F.sxz[at(2 - m)] = -F.sxz[at(1 + m)];
-            }
-        } else {
-            for (int m = 1; m <= nk; ++m) {
-                F.vx[at(1 - m)] = F.vx[at(1 + m)];
-                F.vy[at(1 - m)] = F.vy[at(1 + m)];
-                F.vz[at(2 - m)] = F.vz[at(1 + m)];
-            }
-        }
-    }
-}
-
 // Source injection of step t (add_source, module_wavefield.f90:1115-1228):
 // forces into vx, vy, vz, explosions into sxx, syy, szz; one block per shot,
 // taps grouped by (field, cell) in source order.
@@ -551,13 +538,16 @@ __global__ __launch_bounds__(1024) void ke_inject(const ShotE* __restrict__ shot
 // shot's 3 nr components to a block.  The taps of a box are summed z, y, x
 // outermost to innermost as OWL lists them; a tap of zero weight, which OWL
 // leaves out, adds +0 (its cell may lie outside the grid and is not read).
+// With the free surface a tap above it reads the mirrored plane (vx, vy of
+// k <= 0 that of 2-k, vz of k <= 1 that of 3-k:
+// submodule_forward_modeling.f90:64-73).
 constexpr int kBoxTaps = (2 * kNkw + 1) * (2 * kNkw + 1) * (2 * kNkw + 1);
 constexpr int kRecGroup = kOrderedTaps / kBoxTaps;
 
 __global__ __launch_bounds__(kOrderedThreads) void ke_record(const ShotE* __restrict__ shots, EF F,
                                                              const RecBox* __restrict__ boxes,
                                                              const float* __restrict__ rec_w, float* traces, int nt,
-                                                             int t) {
+                                                             int t, int fs) {
     constexpr int K = 2 * kNkw + 1;
     const ShotE S = shots[blockIdx.y];
     const int r0 = int(blockIdx.x) * kRecGroup, r1 = min(r0 + kRecGroup, 3 * S.nr);
@@ -570,7 +560,9 @@ __global__ __launch_bounds__(kOrderedThreads) void ke_record(const ShotE* __rest
             const float w1 = B.w[0][kx], w2 = B.w[1][ky], w3 = B.w[2][kz];
             if (w1 == 0.f || w2 == 0.f || w3 == 0.f) return 0.0f;
             const float* f = r < S.nr ? F.vx : (r < 2 * S.nr ? F.vy : F.vz);
-            return f[B.cell0 + kx + (long long)ky * S.px + (long long)kz * S.pxy] * w1 * w2 * w3;
+            const int two = r < 2 * S.nr ? 2 : 3, k1 = B.kz0 + kz;  // planes k1 < two - 1 mirror onto two - k1
+            const int dk = fs && k1 < two - 1 ? two - k1 - B.kz0 : kz;
+            return f[B.cell0 + kx + (long long)ky * S.px + (long long)dk * S.pxy] * w1 * w2 * w3;
         },
         [](int) { return 0.0f; }, [&](int r) { return rec_w[S.rec0 + r % S.nr]; },
         [&](int r, float acc) {
@@ -1200,6 +1192,7 @@ void plan_e(owl_elastic3d* b, const owl_acoustic_config* cfg, const float* vp, c
                 const long long lo = 1 - b->pml - b->R;
                 B.cell0 = S.off + (gx[c] - kNkw - lo) + (gy[c] - kNkw - lo) * (long long)S.px +
                           (gz[c] - kNkw - lo) * S.pxy;
+                B.kz0 = gz[c] - kNkw;
                 for (int k = 0; k < 2 * kNkw + 1; ++k) {
                     B.w[0][k] = wx[c][k];
                     B.w[1][k] = wy[c][k];
@@ -1374,24 +1367,18 @@ void maybe_collect(owl_elastic3d* b) {
 }
 
 // One time step of the wavefields F (memory variables in F) into O (O may
-// be F's own fields): [free surface: zero v above it] -> stresses ->
-// [mirror stresses] -> velocities (module_wavefield.f90:52-1090).
+// be F's own fields): stresses -> velocities (module_wavefield.f90:52-1090).
 template <int R>
 void step_e(owl_elastic3d* b, const EF& F, const EV& O, float dt, double bs, double bv) {
     hipStream_t st = b->stream;
-    const unsigned nshot = unsigned(b->sd.size());
     if (64 * b->cy > 256) fail(OWL_ERR_ARG, "launch shape exceeds the sweeps' 256-thread blocks");
     const int ntile = int(b->tile_shot.size());
     const dim3 blk(64, unsigned(b->cy)), grd(unsigned((ntile + 7) / 8 * 8));
     const EM M = media(b);
-    if (b->fs) hipLaunchKernelGGL(ke_surface<R>, dim3(256, nshot), dim3(256), 0, st, b->d_shots.get(), F, b->pml, 0);
     int ev = b->prof.begin(st, 0, bs);
     hipLaunchKernelGGL(ke_stress<R>, grd, blk, 0, st, b->d_shots.get(), b->d_tile_shot.get(), F, O, M, b->d_prof.get(),
                        b->coef, dt, b->idx, b->idy, b->idz, b->pml, b->kc, b->fs, ntile);
     b->prof.end(st, ev);
-    if (b->fs)
-        hipLaunchKernelGGL(ke_surface<R>, dim3(256, nshot), dim3(256), 0, st, b->d_shots.get(), with_fields(F, O),
-                           b->pml, 1);
     ev = b->prof.begin(st, 1, bv);
     hipLaunchKernelGGL(ke_velocity<R>, grd, blk, 0, st, b->d_shots.get(), b->d_tile_shot.get(), F, O, M,
                        b->d_prof.get(), b->coef, dt, b->idx, b->idy, b->idz, b->pml, b->kc, b->fs, ntile);
@@ -1428,26 +1415,17 @@ void run_forward_e(owl_elastic3d* b, bool save_boundary) {
     sweep_bytes(b, bs, bv);
     const unsigned rg = unsigned(std::max(1, (3 * b->max_nr + kRecGroup - 1) / kRecGroup));
     // step t: [boundary record of the state at the start of the step] ->
-    // [free surface: mirror v above it] -> record(t) -> update -> source
+    // record(t) -> update -> source
     auto loop = [&] {
         for (int t = 1; t <= b->nt; ++t) {
             if (save_boundary) strips_e(b, R, F.vx, F.vy, F.vz, t, 1);
-            if (b->fs)
-                hipLaunchKernelGGL(ke_surface<R>, dim3(256, nshot), dim3(256), 0, st, b->d_shots.get(), F, b->pml, 2);
             int ev = b->prof.begin(st, 2, 0);
-            hipLaunchKernelGGL(ke_record, dim3(rg, nshot), dim3(kOrderedThreads), 0, st, b->d_shots.get(), F, b->d_rec_box.get(),
-                               b->d_rec_w.get(), b->d_traces.get(), b->nt, t);
+            hipLaunchKernelGGL(ke_record, dim3(rg, nshot), dim3(kOrderedThreads), 0, st, b->d_shots.get(), F,
+                               b->d_rec_box.get(), b->d_rec_w.get(), b->d_traces.get(), b->nt, t, b->fs);
             b->prof.end(st, ev);
-            if (t == b->nt) {
-                // the last update changes nothing that is recorded; the state
-                // at the start of step nt is the reverse pass's final state,
-                // whose velocities above a free surface are zero (the mirror
-                // undone)
-                if (b->fs)
-                    hipLaunchKernelGGL(ke_surface<R>, dim3(256, nshot), dim3(256), 0, st, b->d_shots.get(), F, b->pml,
-                                       3);
-                break;
-            }
+            // the last update changes nothing that is recorded; the state at the
+            // start of step nt is the reverse pass's final state
+            if (t == b->nt) break;
             step_e<R>(b, F, out_of(F), b->dt, bs, bv);
             // outside every source's active steps the injection would change nothing
             if (t >= b->src_t0 && t <= b->src_t1) {
