@@ -253,7 +253,7 @@ __device__ __forceinline__ void addo(double* base, unsigned off8, double v) {
 template <int R>
 __global__ __launch_bounds__(256) void k_step_fused(const Shot* __restrict__ shots,
                                                     const int* __restrict__ ftile_shot, int nftile,
-                                                    FieldSet F, const float* __restrict__ bk,
+                                                    Sets sets, const float* __restrict__ bk,
                                                     const float* __restrict__ rho,
                                                     const float* __restrict__ prof, Coef c, float dt,
                                                     float idx, float idz, int pml, int zc) {
@@ -263,6 +263,7 @@ __global__ __launch_bounds__(256) void k_step_fused(const Shot* __restrict__ sho
     // the per-row PML coefficients come through scalar loads
     const int tile = __builtin_amdgcn_readfirstlane(xcd_block() * int(blockDim.y) + int(threadIdx.y));
     if (tile >= nftile) return;
+    const FieldSet F = sets.s[blockIdx.y];
     const Shot S = shots[ftile_shot[tile]];
     const int lt = tile - S.ftile0;
     const int tx = lt % S.fntx, tz = lt / S.fntx;
@@ -1369,6 +1370,7 @@ struct owl_acoustic2d {
     DevBuf<float> d_model_in;           // vp, rho of a new model on their way in
     DevBuf<float> fA[3], fB[3], fM[4];  // forward field (ping-pong) and PML memory
     DevBuf<float> aF[3], aM[4];         // adjoint field and PML memory
+    DevBuf<float> aB[3], aM2[4];        // the other half of its ping-pong (fused reverse steps)
     DevBuf<float> d_amp;                // source amplitude rows [row][nt]
     DevBuf<int> d_inj_beg, d_adj_beg, d_rec_beg;
     DevBuf<Tap> d_inj_taps;
@@ -1890,25 +1892,6 @@ void plan(owl_acoustic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     upload_model(b);
 }
 
-FieldSet in_place(float* p, float* vx, float* vz, float* const* m) {
-    FieldSet F{};
-    F.p_in = F.p_out = p;
-    F.vx_in = F.vx_out = vx;
-    F.vz_in = F.vz_out = vz;
-    for (int k = 0; k < 4; ++k) {
-        F.m_in[k] = m[k];
-        F.m_out[k] = m[k];
-    }
-    return F;
-}
-
-Sets one_set(float* p, float* vx, float* vz, float* const* m) {
-    Sets S{};
-    S.s[0] = in_place(p, vx, vz, m);
-    S.s[1] = S.s[0];
-    return S;
-}
-
 enum KernelKind { kKP = 0, kKV = 1, kKPost = 2, kKImage = 3, kKStrips = 4, kKAdj = 5, kKMisfit = 6, kKMerge = 7,
                   kKP2 = 8, kKV2 = 9, kKFused = 13, kKinds = 16 };
 
@@ -1990,6 +1973,19 @@ void launch_step(owl_acoustic2d* b, const Sets& sets, int nsets, float dt) {
     prof_end(b, ev);
 }
 
+double fused_bytes(const owl_acoustic2d* b);
+bool adj_fused(const owl_acoustic2d* b);
+
+// The fused step of nsets field sets, every input distinct from every output.
+template <int R>
+void launch_fused(owl_acoustic2d* b, const Sets& sets, int nsets, float dt) {
+    const int ev = prof_begin(b, kKFused, b->profiling ? nsets * fused_bytes(b) : 0.0);
+    hipLaunchKernelGGL(k_step_fused<R>, dim3(unsigned((b->nftile + 3) / 4), unsigned(nsets)), dim3(64, 4), 0, b->stream,
+                       b->d_shots.get(), b->d_ftile_shot.get(), b->nftile, sets, b->d_bk.get(), b->d_rho.get(),
+                       b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, b->fzc);
+    prof_end(b, ev);
+}
+
 // The source of step t and, unless null, the receivers (and boundary record)
 // of step t+1.  Outside every source's active steps the injection would
 // change nothing and is not launched.
@@ -2022,28 +2018,81 @@ void launch_inject_adjoint(owl_acoustic2d* b, float* pr, int t) {
     prof_end(b, ev);
 }
 
+// One field set's pointers: p, vx, vz and the four PML memory arrays.
+struct SetPtr {
+    float* f[7];
+};
+SetPtr set_of(DevBuf<float>* f, DevBuf<float>* m) {
+    return SetPtr{{f[0].get(), f[1].get(), f[2].get(), m[0].get(), m[1].get(), m[2].get(), m[3].get()}};
+}
+// A step's field set from `in` to `out`, the memory variables to `mout`
+// (in place where they are in's own).
+FieldSet field_set(const SetPtr& in, const SetPtr& out, const SetPtr& mout) {
+    FieldSet F{};
+    F.p_in = in.f[0];
+    F.p_out = out.f[0];
+    F.vx_in = in.f[1];
+    F.vx_out = out.f[1];
+    F.vz_in = in.f[2];
+    F.vz_out = out.f[2];
+    for (int k = 0; k < 4; ++k) {
+        F.m_in[k] = in.f[3 + k];
+        F.m_out[k] = mout.f[3 + k];
+    }
+    return F;
+}
+// Whether the arrays of a fused step's second field sets may be added: the
+// static scratch is sized for the sweeps, and a batch that fills the device
+// without them keeps the sweeps too (twice the room, for the buffers of a
+// reverse pass after a forward run).
+bool room_for(owl_acoustic2d* b, std::initializer_list<const DevBuf<float>*> f) {
+    if (b->borrowed_stream || tl_arena) return false;
+    size_t n = 0, freeb = 0, total = 0;
+    for (const auto* d : f) n += d->size() != b->field_elems;
+    if (n == 0) return true;
+    OWL_HIP(hipMemGetInfo(&freeb, &total));
+    return 2 * n * (b->field_elems * sizeof(float) + (size_t(2) << 20)) < freeb;
+}
+void alloc_zero(owl_acoustic2d* b, DevBuf<float>* f, int n) {
+    for (int k = 0; k < n; ++k) {
+        f[k].alloc(b->field_elems);
+        f[k].zero(b->stream);
+    }
+}
+
 template <int R>
 void run_forward(owl_acoustic2d* b, bool save) {
     hipStream_t st = b->stream;
     b->have_store = false;  // the working sets below hold a stored exact-adjoint state
     b->store_id = 0;
-    for (int k = 0; k < 3; ++k) b->fA[k].zero(st);
-    for (int k = 0; k < 4; ++k) b->fM[k].zero(st);
+    alloc_zero(b, b->fA, 3);
+    alloc_zero(b, b->fM, 4);
     b->d_traces.zero(st);
     if (save) {
         b->d_strips.alloc(b->strip_elems);
         b->d_strips.zero(st);
     }
-    float* m[4] = {b->fM[0].get(), b->fM[1].get(), b->fM[2].get(), b->fM[3].get()};
-    const Sets sets = one_set(b->fA[0].get(), b->fA[1].get(), b->fA[2].get(), m);
+    const bool fused = adj_fused(b) && room_for(b, {&b->fB[0], &b->fB[1], &b->fB[2], &b->fM2[0], &b->fM2[1],
+                                                    &b->fM2[2], &b->fM2[3]});
+    if (fused) {
+        alloc_zero(b, b->fB, 3);
+        alloc_zero(b, b->fM2, 4);
+    }
+    const SetPtr A = set_of(b->fA, b->fM), C = fused ? set_of(b->fB, b->fM2) : A;
     OWL_HIP(hipEventRecord(b->ev0, st));
     // steps 1..nt-1; the update and source of step nt change nothing that
     // OWL records, and skipping them leaves the state of the start of step nt
-    // (OWL's output_final_step_wavefield) in place.
+    // (OWL's output_final_step_wavefield) in place: in fA, where an even
+    // number of fused steps ends if it starts there.
+    int cur = fused ? (b->nt - 1) % 2 : 0;
     for (int t = 1; t <= b->nt - 1; ++t) {
-        launch_step<R>(b, sets, 1, b->dt);
-        float* f[3] = {b->fA[0].get(), b->fA[1].get(), b->fA[2].get()};
-        post_step<R>(b, f, t, b->d_traces.get(), save ? b->d_strips.get() : nullptr);
+        const SetPtr &in = cur ? C : A, &out = cur ? A : C;
+        Sets sets{};
+        sets.s[0] = sets.s[1] = field_set(in, out, out);
+        if (fused) launch_fused<R>(b, sets, 1, b->dt);
+        else launch_step<R>(b, sets, 1, b->dt);
+        cur = 1 - cur;
+        post_step<R>(b, out.f, t, b->d_traces.get(), save ? b->d_strips.get() : nullptr);
     }
     OWL_HIP(hipGetLastError());
     OWL_HIP(hipEventRecord(b->ev1, st));
@@ -2058,6 +2107,10 @@ void run_forward(owl_acoustic2d* b, bool save) {
 }
 
 // OWL's reverse loop t = nt .. hnt (submodule_fwi_gradient.f90:75-167).
+// Where the fused step may run (adj_fused) both field sets advance by it, out
+// of place with their memory variables: one launch of 156 us for 32 shots of 461 x 461 nodes in
+// place of 254 us of sweeps.  (Running 10 or 16 of the shots at a time, so
+// that a step finds its fields in the last-level cache, gained nothing.)
 template <int R>
 void run_reverse_owl(owl_acoustic2d* b) {
     hipStream_t st = b->stream;
@@ -2065,17 +2118,10 @@ void run_reverse_owl(owl_acoustic2d* b) {
     b->store_id = 0;
     if (!b->have_boundary || !b->fwd_state_valid)
         fail(OWL_ERR_STATE, "the adjoint needs a preceding forward run with boundary saving");
-    for (int k = 0; k < 3; ++k) {
-        b->fB[k].alloc(b->field_elems);
-        b->fB[k].zero(st);
-        b->aF[k].alloc(b->field_elems);
-        b->aF[k].zero(st);
-    }
-    for (int k = 0; k < 4; ++k) {
-        b->fM[k].zero(st);
-        b->aM[k].alloc(b->field_elems);
-        b->aM[k].zero(st);
-    }
+    alloc_zero(b, b->fB, 3);
+    alloc_zero(b, b->fM, 4);
+    alloc_zero(b, b->aF, 3);
+    alloc_zero(b, b->aM, 4);
     b->d_edge.alloc(std::max<size_t>(b->edge_elems, 1));
     b->d_gv.alloc(b->grad_elems);
     b->d_gr.alloc(b->grad_elems);
@@ -2086,44 +2132,49 @@ void run_reverse_owl(owl_acoustic2d* b) {
         b->d_energy.zero(st);
     }
     const unsigned nshot = unsigned(b->sd.size());
+    const bool fused = adj_fused(b) && room_for(b, {&b->fM2[0], &b->fM2[1], &b->fM2[2], &b->fM2[3], &b->aB[0],
+                                                    &b->aB[1], &b->aB[2], &b->aM2[0], &b->aM2[1], &b->aM2[2],
+                                                    &b->aM2[3]});
+    if (fused) {
+        alloc_zero(b, b->fM2, 4);
+        alloc_zero(b, b->aB, 3);
+        alloc_zero(b, b->aM2, 4);
+    }
+    const SetPtr fw[2] = {set_of(b->fA, b->fM), set_of(b->fB, fused ? b->fM2 : b->fM)};
+    const SetPtr aw[2] = {set_of(b->aF, b->aM), fused ? set_of(b->aB, b->aM2) : set_of(b->aF, b->aM)};
+    const int cc = b->cfg.cc_step_interval > 0 ? b->cfg.cc_step_interval : 1;
+    const unsigned ig = unsigned(std::max(1, std::min(1024, (int)((b->grad_elems / nshot + 255) / 256))));
+    // imaging: p, prev p, pr, rho*vp^3 and six velocity fields read once
+    // (40 B/point), two FP64 accumulators read and written (32 B/point)
+    const double image_bytes = 72.0 * double(b->grad_elems);
     // OWL loops down to the first source's hnt of each shot; a batch whose
     // shots disagree runs down to the smallest one and images each shot only
     // while t >= its own hnt (the extra reverse steps of the other shots
     // touch no gradient).
     int hnt = b->nt;
     for (auto& H : b->hs) hnt = std::min(hnt, std::max(H.hnt, 1));
-    DevBuf<float>* A = b->fA;
-    DevBuf<float>* B = b->fB;
-    const int cc = b->cfg.cc_step_interval > 0 ? b->cfg.cc_step_interval : 1;
-    const unsigned ig = unsigned(std::max(1, std::min(1024, (int)((b->grad_elems / nshot + 255) / 256))));
-    // imaging: p, prev p, pr, rho*vp^3 and six velocity fields read once
-    // (40 B/point), two FP64 accumulators read and written (32 B/point)
-    const double image_bytes = 72.0 * double(b->grad_elems);
     OWL_HIP(hipEventRecord(b->ev0, st));
+    int cur = 0;
     for (int t = b->nt; t >= hnt; --t) {
+        const SetPtr &A = fw[cur], &B = fw[1 - cur], &a = aw[cur], &r = aw[1 - cur];
         int ev = prof_begin(b, kKStrips);
-        hipLaunchKernelGGL(k_inject_strips<R>, dim3(16, nshot), dim3(256), 0, st, b->d_shots.get(),
-                           A[1].get(), A[2].get(), b->d_strips.get(), b->d_edge.get(), t, b->pml);
+        hipLaunchKernelGGL(k_inject_strips<R>, dim3(16, nshot), dim3(256), 0, st, b->d_shots.get(), A.f[1], A.f[2],
+                           b->d_strips.get(), b->d_edge.get(), t, b->pml);
         prof_end(b, ev);
         Sets sets{};
-        float* fm[4] = {b->fM[0].get(), b->fM[1].get(), b->fM[2].get(), b->fM[3].get()};
-        float* am[4] = {b->aM[0].get(), b->aM[1].get(), b->aM[2].get(), b->aM[3].get()};
-        sets.s[0] = in_place(A[0].get(), A[1].get(), A[2].get(), fm);
-        sets.s[0].p_out = B[0].get();
-        sets.s[0].vx_out = B[1].get();
-        sets.s[0].vz_out = B[2].get();
-        sets.s[1] = in_place(b->aF[0].get(), b->aF[1].get(), b->aF[2].get(), am);
-        launch_step<R>(b, sets, 2, -b->dt);
-        launch_inject_adjoint(b, b->aF[0].get(), t);
+        sets.s[0] = field_set(A, B, B);
+        sets.s[1] = field_set(a, r, r);
+        if (fused) launch_fused<R>(b, sets, 2, -b->dt);
+        else launch_step<R>(b, sets, 2, -b->dt);
+        launch_inject_adjoint(b, r.f[0], t);
         ev = prof_begin(b, kKImage, (t % cc == 0) ? image_bytes : 0.0);
         if (t % cc == 0)
-            hipLaunchKernelGGL(k_image_owl<R>, dim3(ig, nshot), dim3(256), 0, st, b->d_shots.get(),
-                               B[0].get(), B[1].get(), B[2].get(), A[0].get(), A[1].get(), A[2].get(),
-                               b->d_edge.get(), b->aF[0].get(), b->aF[1].get(), b->aF[2].get(),
+            hipLaunchKernelGGL(k_image_owl<R>, dim3(ig, nshot), dim3(256), 0, st, b->d_shots.get(), B.f[0], B.f[1],
+                               B.f[2], A.f[0], A.f[1], A.f[2], b->d_edge.get(), r.f[0], r.f[1], r.f[2],
                                b->d_den.get(), b->d_gv.get(), b->d_gr.get(), t == b->nt ? 1 : 0, b->pml,
                                b->energy_precond ? b->d_energy.get() : nullptr, b->grad_elems, t);
         prof_end(b, ev);
-        std::swap(A, B);
+        cur = 1 - cur;
     }
     if (b->energy_precond)
         hipLaunchKernelGGL(k_energy_precond, dim3(nshot), dim3(256), 0, st, b->d_shots.get(), b->d_gv.get(),
@@ -2132,15 +2183,11 @@ void run_reverse_owl(owl_acoustic2d* b) {
     OWL_HIP(hipEventRecord(b->ev1, st));
     OWL_HIP(hipStreamSynchronize(st));
     prof_collect(b);
-    // the forward state now lives in whichever buffer A points to; the
-    // boundary records have been consumed
-    if (A != b->fA)
-        for (int k = 0; k < 3; ++k) std::swap(b->fA[k], b->fB[k]);
     float ms = 0.f;
     OWL_HIP(hipEventElapsedTime(&ms, b->ev0, b->ev1));
     b->last_ms = ms;
     b->last_updates = 2.0 * double(b->nt - hnt + 1) * b->pts_full;
-    b->fwd_state_valid = false;
+    b->fwd_state_valid = false;  // fA, fB hold the reverse pass's states
 }
 
 
@@ -2223,15 +2270,8 @@ void fwd_step(owl_acoustic2d* b, const W7& in, const W7& out, int t, bool record
         F.m_out[k] = out.f[3 + k];
     }
     sets.s[1] = F;
-    if (use_fused(b, in, out)) {
-        const int ev = prof_begin(b, kKFused, b->profiling ? fused_bytes(b) : 0.0);
-        hipLaunchKernelGGL(k_step_fused<R>, dim3(unsigned((b->nftile + 3) / 4)), dim3(64, 4), 0, b->stream,
-                           b->d_shots.get(), b->d_ftile_shot.get(), b->nftile, F, b->d_bk.get(), b->d_rho.get(),
-                           b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, b->fzc);
-        prof_end(b, ev);
-    } else {
-        launch_step<R>(b, sets, 1, b->dt);
-    }
+    if (use_fused(b, in, out)) launch_fused<R>(b, sets, 1, b->dt);
+    else launch_step<R>(b, sets, 1, b->dt);
     post_step<R>(b, out.f, t, record ? b->d_traces.get() : nullptr, nullptr);
 }
 
@@ -2845,6 +2885,8 @@ void autotune_rows(owl_acoustic2d* b) {
         F.m_in[k] = in.f[3 + k];
         F.m_out[k] = out.f[3 + k];
     }
+    Sets sets{};
+    sets.s[0] = sets.s[1] = F;
     DevBuf<float>* a = b->adj;
     DevBuf<float>* a2 = b->adj2;
     const AdjIO io{a[0].get(), a[3].get(), a[4].get(), a[7].get(), a[8].get(),
@@ -2868,7 +2910,7 @@ void autotune_rows(owl_acoustic2d* b) {
         upload_fused_tiling(b);
         const float ms = timed([&] {
             hipLaunchKernelGGL(k_step_fused<R>, dim3(unsigned((b->nftile + 3) / 4)), dim3(64, 4), 0, st,
-                               b->d_shots.get(), b->d_ftile_shot.get(), b->nftile, F, b->d_bk.get(), b->d_rho.get(),
+                               b->d_shots.get(), b->d_ftile_shot.get(), b->nftile, sets, b->d_bk.get(), b->d_rho.get(),
                                b->d_prof.get(), b->coef, b->dt, b->idx, b->idz, b->pml, b->fzc);
         });
         if (ms < tf) tf = ms, best_f = z;
