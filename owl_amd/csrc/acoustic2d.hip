@@ -2108,9 +2108,10 @@ void run_forward(owl_acoustic2d* b, bool save) {
 
 // OWL's reverse loop t = nt .. hnt (submodule_fwi_gradient.f90:75-167).
 // Where the fused step may run (adj_fused) both field sets advance by it, out
-// of place with their memory variables: one launch of 156 us for 32 shots of 461 x 461 nodes in
-// place of 254 us of sweeps.  (Running 10 or 16 of the shots at a time, so
-// that a step finds its fields in the last-level cache, gained nothing.)
+// of place with their memory variables: one launch of 156 us for 32 shots of
+// 461 x 461 nodes in place of 254 us of sweeps.  (Running 10 or 16 of the
+// shots at a time, so that a step finds its fields in the last-level cache,
+// gained nothing.)
 template <int R>
 void run_reverse_owl(owl_acoustic2d* b) {
     hipStream_t st = b->stream;

@@ -580,6 +580,154 @@ __global__ void k2e_merge(const ShotE2* __restrict__ shots, const int* __restric
     }
 }
 
+// Free surface: where shot s's columns lie in the buffers of k2e_fs_columns.
+struct FsColumns {
+    long long rho0, dp0, map0, win0;  // mapped density, work, mapped values, window gradients
+    int zi0, tab0, nx, nz0;           // row depths, spline tables; window size
+};
+
+// Free surface: the accumulators' columns on the refined rows to the window's
+// rows (map_irregular_to_regular, module_vars.f90:175-203): the natural cubic
+// spline through z_i, A, B, C (blockIdx.z = 0..2) through rows 1 .. nz and
+// rho x 1e-3 (3) through all rows -pml .. nz+pml+1.  One thread per column,
+// values [row][column], so that a wavefront reads a row's 64 columns at once;
+// rows come 8 at a time, ahead of the two serial passes.  tab: the part of
+// the elimination that the depths alone decide (fsm::spline_table).  Bound by
+// its serial FP64 divisions: 296 us for 8 shots of 301 x 201 nodes, which
+// took 26 ms column by column on the host.
+__global__ __launch_bounds__(64) void k2e_fs_columns(const ShotE2* __restrict__ shots,
+                                                     const FsColumns* __restrict__ cols, int s0,
+                                                     const double* __restrict__ gA, const double* __restrict__ gB,
+                                                     const double* __restrict__ gC, const float* __restrict__ rho,
+                                                     const float* __restrict__ zi, const double* __restrict__ tab,
+                                                     double* __restrict__ work, double* __restrict__ map, int pml,
+                                                     float dz) {
+    constexpr int U = 8;
+    const int s = s0 + int(blockIdx.y), q = int(blockIdx.z);
+    const FsColumns C = cols[s];
+    const int col = int(blockIdx.x) * 64 + int(threadIdx.x), nx = C.nx;
+    if (col >= nx) return;
+    const int nzr = shots[s].nz, n = q < 3 ? nzr : nzr + 2 * pml + 2;
+    const float* x = zi + C.zi0 + (q < 3 ? pml + 1 : 0);
+    const double* cp = tab + C.tab0 + (q < 3 ? 0 : 2 * nzr);
+    const double* den = cp + n;
+    const double* g = (q == 0 ? gA : q == 1 ? gB : gC) + size_t(shots[s].g0) + col;
+    const float* rg = rho + C.rho0 + col;
+    const long long base = cols[s0].dp0;
+    double* M = work + (C.dp0 - base) + size_t(q) * nzr * nx + col;
+    double* out = map + (C.map0 - cols[s0].map0) + size_t(q) * C.nz0 * nx + col;
+    auto val = [&](int i) { return q < 3 ? g[size_t(i) * nx] : double(rg[size_t(i) * nx] * 1.0e-3f); };
+    // elimination: dp of rows 1 .. n-2, kept where M will be
+    double gm = val(0), gc = val(1), dp = 0.0;
+    M[0] = 0.0;
+    M[size_t(n - 1) * nx] = 0.0;
+    for (int i0 = 1; i0 < n - 1; i0 += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = val(min(i0 + u + 1, n - 1));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u;
+            if (i < n - 1) {
+                const double h0 = double(x[i]) - x[i - 1], h1 = double(x[i + 1]) - x[i];
+                const double r = 6.0 * ((v[u] - gc) / h1 - (gc - gm) / h0);
+                dp = (r - h0 * dp) / den[i];
+                M[size_t(i) * nx] = dp;
+                gm = gc;
+                gc = v[u];
+            }
+        }
+    }
+    // back substitution
+    double m = 0.0;
+    for (int i0 = n - 2; i0 >= 1; i0 -= U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = M[size_t(max(i0 - u, 1)) * nx];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 - u;
+            if (i >= 1) {
+                m = v[u] - cp[i] * m;
+                M[size_t(i) * nx] = m;
+            }
+        }
+    }
+    int seg = 0;  // x[seg] <= v < x[seg + 1], the end segments beyond the ends
+    for (int k = 0; k < C.nz0; ++k) {
+        const float v = float(k) * dz;
+        while (seg < n - 2 && x[seg + 1] <= v) ++seg;
+        const double h = double(x[seg + 1]) - x[seg];
+        const double A = (double(x[seg + 1]) - v) / h, B = (double(v) - x[seg]) / h;
+        const size_t a = size_t(seg) * nx, b = a + size_t(nx);
+        out[size_t(k) * nx] = A * val(seg) + B * val(seg + 1) +
+                              ((A * A * A - A) * M[a] + (B * B * B - B) * M[b]) * h * h / 6.0;
+    }
+}
+
+// Chain rule (submodule_fwi_gradient.f90:330-360) with vp, vs in km/s and
+// rho in g/cm^3: grad_vp = 2 rho vp A, grad_vs = 2 rho vs B, grad_rho = C.
+__host__ __device__ inline void chain_rule2r(float vp, float vs, double r, double A, double B, double C, double& gv,
+                                             double& gs, double& gr) {
+    const double p = double(vp * 1.0e-3f), v = double(vs * 1.0e-3f);
+    gv = 2.0 * r * p * A;
+    gs = 2.0 * r * v * B;
+    gr = C;
+}
+
+// The mapped values of window node (i, k) through the chain rule with the
+// shot's own mapped density and the model's vp, vs at model node m.
+__device__ __forceinline__ void fs_chain(const FsColumns& C, const double* __restrict__ map, long long map0, int i,
+                                         int k, float vp, float vs, double& gv, double& gs, double& gr) {
+    const size_t o = size_t(C.map0 - map0) + size_t(k) * C.nx + size_t(i), n = size_t(C.nx) * C.nz0;
+    chain_rule2r(vp, vs, double(float(map[o + 3 * n])), map[o], map[o + n], map[o + 2 * n], gv, gs, gr);
+}
+
+// Adds shots s0 .. s1 - 1, in order, to the gradients on the full model.
+__global__ void k2e_fs_merge(const FsColumns* __restrict__ cols, const int* __restrict__ win, int s0, int s1,
+                             const double* __restrict__ map, const float* __restrict__ vp,
+                             const float* __restrict__ vs, double* gv, double* gs, double* gr, int nx, int nz) {
+    const long long n = (long long)nx * nz, map0 = cols[s0].map0;
+    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < n;
+         e += (long long)gridDim.x * blockDim.x) {
+        const int kz = int(e % nz), ix = int(e / nz);
+        double a = gv[e], b = gs[e], c = gr[e];
+        for (int s = s0; s < s1; ++s) {
+            const int i = ix - (win[2 * s] - 1), k = kz - (win[2 * s + 1] - 1);
+            if (i < 0 || i >= cols[s].nx || k < 0 || k >= cols[s].nz0) continue;
+            double x, y, z;
+            fs_chain(cols[s], map, map0, i, k, vp[e], vs[e], x, y, z);
+            a += x;
+            b += y;
+            c += z;
+        }
+        gv[e] = a;
+        gs[e] = b;
+        gr[e] = c;
+    }
+}
+
+// Shots s0 + blockIdx.y on their windows, z fastest, NaN/Inf -> 0.
+__global__ void k2e_fs_window(const FsColumns* __restrict__ cols, const int* __restrict__ win, int s0,
+                              const double* __restrict__ map, const float* __restrict__ vp,
+                              const float* __restrict__ vs, float* __restrict__ gv, float* __restrict__ gs,
+                              float* __restrict__ gr, int nz) {
+    const int s = s0 + int(blockIdx.y);
+    const FsColumns C = cols[s];
+    const long long n = (long long)C.nx * C.nz0;
+    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < n;
+         e += (long long)gridDim.x * blockDim.x) {
+        const int k = int(e % C.nz0), i = int(e / C.nz0);
+        const size_t m = size_t(win[2 * s + 1] - 1 + k) + size_t(win[2 * s] - 1 + i) * size_t(nz);
+        double x, y, z;
+        fs_chain(C, map, cols[s0].map0, i, k, vp[m], vs[m], x, y, z);
+        const float a = float(x), b = float(y), c = float(z);
+        gv[C.win0 + e] = isfinite(a) ? a : 0.0f;
+        gs[C.win0 + e] = isfinite(b) ? b : 0.0f;
+        gr[C.win0 + e] = isfinite(c) ? c : 0.0f;
+    }
+}
+
 struct ShotHostE2 {
     int id = 0, nx = 0, nz = 0, nxbeg = 1, nzbeg = 1, hnt = 1;
     float ox = 0, oz = 0;
@@ -598,7 +746,11 @@ struct owl_elastic2d {
     bool fs = false;                       // OWL's free surface on the depth-refined mesh
     float fs_refine = 4.0f, fs_dzmax = 0.0f;
     std::vector<owl::fsm::SsgMesh> mesh;   // per shot (free surface)
-    std::vector<std::vector<float>> rho_map;  // per shot: rho on the refined rows, column i (1..nx) at [(i-1) nrj + j + pml]
+    std::vector<FsColumns> cols;              // per shot (free surface)
+    DevBuf<FsColumns> d_cols;
+    DevBuf<float> d_rho_map, d_zi, d_vp, d_vs;  // rho on the refined rows [row][column], z_i; the model
+    DevBuf<double> d_spline, d_fs_work, d_fs_map;
+    DevBuf<float> d_fs_win;
     int R = 4, pml = 15, nt = 0, kc = 0, cy = 4;  // kc: rows per tile, set by the plan if 0
     float dt = 0, idx = 0, idz = 0;
     e2::Coef coef{};
@@ -764,7 +916,10 @@ void plan2(owl_elastic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     b->src_t1 = -1;
     b->pts_full = 0;
     b->mesh.assign(b->fs ? size_t(nshot) : 0, fsm::SsgMesh{});
-    b->rho_map.assign(b->fs ? size_t(nshot) : 0, std::vector<float>{});
+    b->cols.assign(b->fs ? size_t(nshot) : 0, FsColumns{});
+    std::vector<float> rho_map, zi;
+    std::vector<double> spline;
+    long long fs_dp = 0, fs_map = 0, fs_win = 0;
     // free surface: per shot the window's c11 (= c33), c13, c55 and rho
     // mapped onto the refined rows, column i at [(i + pml) * nrj + j + pml]
     // for i, j = -pml .. n+pml+1
@@ -852,11 +1007,23 @@ void plan2(owl_elastic2d* b, const owl_acoustic_config* cfg, const float* vp, co
             if (cfg->dt > dts)
                 fail(OWL_ERR_CFL, "dt = " + std::to_string(cfg->dt) + " exceeds the stable dt = " +
                                       std::to_string(dts) + " of the free-surface mesh");
-            auto& rm = b->rho_map[size_t(s)];
-            rm.resize(size_t(H.nx) * nrj);
-            for (int i = 1; i <= H.nx; ++i)
-                std::copy(mr.begin() + long(size_t(i + pml) * nrj), mr.begin() + long(size_t(i + pml + 1) * nrj),
-                          rm.begin() + long(size_t(i - 1) * nrj));
+            FsColumns& C = b->cols[size_t(s)];
+            C.nx = H.nx;
+            C.nz0 = H.nz;
+            C.rho0 = (long long)rho_map.size();
+            for (int k = 0; k < nrj; ++k)
+                for (int i = 1; i <= H.nx; ++i) rho_map.push_back(mr[size_t(i + pml) * nrj + size_t(k)]);
+            C.zi0 = int(zi.size());
+            zi.insert(zi.end(), Mh.zi.begin(), Mh.zi.begin() + nrj);
+            C.tab0 = int(spline.size());
+            fsm::spline_table(Mh.zi.data() + pml + 1, nzr, spline);
+            fsm::spline_table(Mh.zi.data(), nrj, spline);
+            C.dp0 = fs_dp;
+            fs_dp += (long long)H.nx * (3 * nzr + nrj);
+            C.map0 = fs_map;
+            fs_map += 4LL * H.nx * H.nz;
+            C.win0 = fs_win;
+            fs_win += (long long)H.nx * H.nz;
             S.sc0 = int(scal.size());
             scal.insert(scal.end(), Mh.sci.begin(), Mh.sci.end());
             scal.insert(scal.end(), Mh.sch.begin(), Mh.sch.end());
@@ -1118,6 +1285,14 @@ void plan2(owl_elastic2d* b, const owl_acoustic_config* cfg, const float* vp, co
     }
     if (scal.empty()) scal.push_back(1.0f);
     b->d_sc.upload(scal, stm);
+    if (b->fs) {
+        b->d_cols.upload(b->cols, stm);
+        b->d_rho_map.upload(rho_map, stm);
+        b->d_zi.upload(zi, stm);
+        b->d_spline.upload(spline, stm);
+        b->d_vp.upload(b->vp_full, stm);
+        b->d_vs.upload(b->vs_full, stm);
+    }
     std::vector<float> mxz(n, 0.f), rx(n, 1.f), rz(n, 1.f);
     for (size_t s = 0; s < b->sd.size(); ++s) {
         const ShotE2& S = b->sd[s];
@@ -1409,54 +1584,43 @@ void traces_to_device2(owl_elastic2d* b, const float* in, DevBuf<float>& dev) {
     OWL_HIP(hipStreamSynchronize(b->stream));
 }
 
-// Chain rule (submodule_fwi_gradient.f90:330-360) with vp, vs in km/s and
-// rho in g/cm^3: grad_vp = 2 rho vp A, grad_vs = 2 rho vs B, grad_rho = C.
-inline void chain_rule2r(float vp, float vs, double r, double A, double B, double C, double& gv, double& gs,
-                         double& gr) {
-    const double p = double(vp * 1.0e-3f), v = double(vs * 1.0e-3f);
-    gv = 2.0 * r * p * A;
-    gs = 2.0 * r * v * B;
-    gr = C;
-}
 inline void chain_rule2(float vp, float vs, float rho, double A, double B, double C, double& gv, double& gs,
                         double& gr) {
     chain_rule2r(vp, vs, double(rho * 1.0e-3f), A, B, C, gv, gs, gr);
 }
 
-// Free surface: shot s's accumulators on its refined rows to the window's
-// rows (map_irregular_to_regular, submodule_fwi_gradient.f90:324-338): A,
-// B, C column by column through z_i(1 .. nz), and rho x 1e-3 through all
-// refined rows -pml .. nz+pml+1; then the chain rule with the window's vp,
-// vs.  Outputs (nz_w, nx_w) z fastest.
-void window_grads_fs(const owl_elastic2d* b, size_t s, const double* gA, const double* gB, const double* gC,
-                     std::vector<double>& gv, std::vector<double>& gs, std::vector<double>& gr) {
-    const ShotE2& S = b->sd[s];
-    const ShotHostE2& H = b->hs[s];
-    const fsm::SsgMesh& M = b->mesh[s];
-    const int nx = H.nx, nz0 = H.nz, nzr = S.nz, pml = b->pml, nrj = nzr + 2 * pml + 2;
-    gv.assign(size_t(nx) * nz0, 0.0);
-    gs.assign(gv.size(), 0.0);
-    gr.assign(gv.size(), 0.0);
-    const size_t nr_ = static_cast<size_t>(nzr), n0 = static_cast<size_t>(nz0), nj = static_cast<size_t>(nrj);
-    std::vector<double> ca(nr_), cb(nr_), cc(nr_), ma(n0), mb(n0), mc(n0), rr(nj), mr(n0);
-    for (int i = 1; i <= nx; ++i) {
-        for (int j = 1; j <= nzr; ++j) {
-            const size_t o = size_t(S.g0) + size_t(i - 1) + size_t(j - 1) * nx;
-            ca[size_t(j - 1)] = gA[o];
-            cb[size_t(j - 1)] = gB[o];
-            cc[size_t(j - 1)] = gC[o];
+// Free surface: maps the accumulators of the shots to their windows' rows, as
+// many shots at a time as 64 MB of work and mapped values hold, and calls
+// use(s0, s1) after shots s0 .. s1 - 1.
+template <class U>
+void map_columns_fs(owl_elastic2d* b, U&& use) {
+    const int nshot = int(b->sd.size()), pml = b->pml;
+    auto work = [&](int s) { return (long long)b->cols[size_t(s)].nx * (4 * b->sd[size_t(s)].nz + 2 * pml + 2); };
+    auto mapped = [&](int s) { return 4LL * b->cols[size_t(s)].nx * b->cols[size_t(s)].nz0; };
+    for (const ShotE2& S : b->sd)
+        if (S.nz < 3) fail(OWL_ERR_ARG, "too few refined rows");
+    for (int pass = 0; pass < 2; ++pass) {  // the largest group's buffers, then the groups
+        size_t wmax = 0, mmax = 0;
+        for (int s0 = 0, s1 = 0; s0 < nshot; s0 = s1) {
+            long long w = 0, m = 0;
+            int nx = 0;
+            for (; s1 < nshot && (s1 == s0 || w + m + work(s1) + mapped(s1) <= (8LL << 20)); ++s1) {
+                w += work(s1);
+                m += mapped(s1);
+                nx = std::max(nx, b->cols[size_t(s1)].nx);
+            }
+            wmax = std::max(wmax, size_t(w));
+            mmax = std::max(mmax, size_t(m));
+            if (pass == 0) continue;
+            hipLaunchKernelGGL(k2e_fs_columns, dim3(unsigned((nx + 63) / 64), unsigned(s1 - s0), 4), dim3(64), 0,
+                               b->stream, b->d_shots.get(), b->d_cols.get(), s0, b->d_gA.get(), b->d_gB.get(),
+                               b->d_gC.get(), b->d_rho_map.get(), b->d_zi.get(), b->d_spline.get(),
+                               b->d_fs_work.get(), b->d_fs_map.get(), pml, b->cfg.dz);
+            use(s0, s1);
+            OWL_HIP(hipGetLastError());
         }
-        fsm::column_to_regular_ssg(M, nz0, ca.data(), ma.data());
-        fsm::column_to_regular_ssg(M, nz0, cb.data(), mb.data());
-        fsm::column_to_regular_ssg(M, nz0, cc.data(), mc.data());
-        const std::vector<float>& rm = b->rho_map[s];
-        for (int k = 0; k < nrj; ++k) rr[size_t(k)] = double(rm[size_t(i - 1) * nrj + k] * 1.0e-3f);
-        fsm::spline_to_regular(M.zi.data(), rr.data(), nrj, M.dz, nz0, mr.data());
-        for (int k = 1; k <= nz0; ++k) {
-            const size_t m = model_index2(b, H, i, k), o = size_t(k - 1) + size_t(i - 1) * nz0;
-            chain_rule2r(b->vp_full[m], b->vs_full[m], double(float(mr[size_t(k - 1)])), ma[size_t(k - 1)],
-                         mb[size_t(k - 1)], mc[size_t(k - 1)], gv[o], gs[o], gr[o]);
-        }
+        b->d_fs_work.alloc(wmax);
+        b->d_fs_map.alloc(mmax);
     }
 }
 
@@ -1509,28 +1673,29 @@ owl_status owl_elastic2d_adjoint(owl_elastic2d* b, const float* adj, float* grad
         if (!b || !adj) fail(OWL_ERR_ARG, "null argument");
         traces_to_device2(b, adj, b->d_adj);
         dispatch_R2e(b->R, [&](auto r) { run_reverse2<decltype(r)::value>(b); });
+        if (b->fs) {
+            const size_t n = size_t(b->cols.back().win0) + size_t(b->cols.back().nx) * b->cols.back().nz0;
+            b->d_fs_win.alloc(3 * n);
+            float* w = b->d_fs_win.get();
+            map_columns_fs(b, [&](int s0, int s1) {
+                hipLaunchKernelGGL(k2e_fs_window, dim3(256, unsigned(s1 - s0)), dim3(256), 0, b->stream,
+                                   b->d_cols.get(), b->d_win.get(), s0, b->d_fs_map.get(), b->d_vp.get(),
+                                   b->d_vs.get(), w, w + n, w + 2 * n, b->cfg.nz);
+            });
+            OWL_HIP(hipStreamSynchronize(b->stream));
+            float* out[3] = {grad_vp, grad_vs, grad_rho};
+            for (int k = 0; k < 3; ++k)
+                if (out[k]) OWL_HIP(hipMemcpy(out[k], w + size_t(k) * n, n * sizeof(float), hipMemcpyDeviceToHost));
+            return;
+        }
         std::vector<double> gA(b->grad_elems), gB(b->grad_elems), gC(b->grad_elems);
         OWL_HIP(hipMemcpy(gA.data(), b->d_gA.get(), gA.size() * sizeof(double), hipMemcpyDeviceToHost));
         OWL_HIP(hipMemcpy(gB.data(), b->d_gB.get(), gB.size() * sizeof(double), hipMemcpyDeviceToHost));
         OWL_HIP(hipMemcpy(gC.data(), b->d_gC.get(), gC.size() * sizeof(double), hipMemcpyDeviceToHost));
         // per-shot window gradients (nz_s, nx_s), z fastest, NaN/Inf -> 0
-        size_t wo = 0;
         for (size_t s = 0; s < b->sd.size(); ++s) {
             const ShotE2& S = b->sd[s];
             const ShotHostE2& H = b->hs[s];
-            if (b->fs) {
-                std::vector<double> gv, gs, gr;
-                window_grads_fs(b, s, gA.data(), gB.data(), gC.data(), gv, gs, gr);
-                for (size_t e = 0; e < gv.size(); ++e) {
-                    const float a = float(gv[e]), c = float(gs[e]), f = float(gr[e]);
-                    if (grad_vp) grad_vp[wo + e] = std::isfinite(a) ? a : 0.f;
-                    if (grad_vs) grad_vs[wo + e] = std::isfinite(c) ? c : 0.f;
-                    if (grad_rho) grad_rho[wo + e] = std::isfinite(f) ? f : 0.f;
-                }
-                wo += gv.size();
-                continue;
-            }
-            wo += size_t(S.nx) * S.nz;
             for (int k = 0; k < S.nz; ++k)
                 for (int i = 0; i < S.nx; ++i) {
                     const size_t src = size_t(S.g0) + i + size_t(k) * S.nx;
@@ -1568,12 +1733,19 @@ owl_status owl_elastic2d_gradient(owl_elastic2d* b, const float* obs, double* mi
                            b->d_scratch.get());
         dispatch_R2e(b->R, [&](auto r) { run_reverse2<decltype(r)::value>(b); });
         const size_t nfull = size_t(b->cfg.nx) * b->cfg.nz;
-        if (!b->fs) {
-            for (auto* g : {&b->d_fA, &b->d_fB, &b->d_fC}) g->alloc(nfull);
-            const unsigned mg = unsigned(std::min<size_t>(8192, (nfull + 255) / 256));
+        for (auto* g : {&b->d_fA, &b->d_fB, &b->d_fC}) g->alloc(nfull);
+        const unsigned mg = unsigned(std::min<size_t>(8192, (nfull + 255) / 256));
+        if (!b->fs)
             hipLaunchKernelGGL(k2e_merge, dim3(mg), dim3(256), 0, st, b->d_shots.get(), b->d_win.get(), int(nshot),
                                b->d_gA.get(), b->d_gB.get(), b->d_gC.get(), b->d_fA.get(), b->d_fB.get(),
                                b->d_fC.get(), b->cfg.nx, b->cfg.nz);
+        else if (grad_vp || grad_vs || grad_rho) {
+            for (auto* g : {&b->d_fA, &b->d_fB, &b->d_fC}) g->zero(st);
+            map_columns_fs(b, [&](int s0, int s1) {
+                hipLaunchKernelGGL(k2e_fs_merge, dim3(mg), dim3(256), 0, st, b->d_cols.get(), b->d_win.get(), s0, s1,
+                                   b->d_fs_map.get(), b->d_vp.get(), b->d_vs.get(), b->d_fA.get(), b->d_fB.get(),
+                                   b->d_fC.get(), b->cfg.nx, b->cfg.nz);
+            });
         }
         OWL_HIP(hipGetLastError());
         OWL_HIP(hipStreamSynchronize(st));
@@ -1582,39 +1754,14 @@ owl_status owl_elastic2d_gradient(owl_elastic2d* b, const float* obs, double* mi
             OWL_HIP(hipMemcpy(m2.data(), b->d_misfit.get(), m2.size() * sizeof(double), hipMemcpyDeviceToHost));
             for (unsigned s = 0; s < nshot; ++s) misfit[s] = m2[2 * s] + m2[2 * s + 1];
         }
-        if (b->fs && (grad_vp || grad_vs || grad_rho)) {
-            // each shot mapped back to its window and through the chain rule
-            // with its own mapped density, then summed on the model
-            std::vector<double> gA(b->grad_elems), gB(b->grad_elems), gC(b->grad_elems);
-            OWL_HIP(hipMemcpy(gA.data(), b->d_gA.get(), gA.size() * sizeof(double), hipMemcpyDeviceToHost));
-            OWL_HIP(hipMemcpy(gB.data(), b->d_gB.get(), gB.size() * sizeof(double), hipMemcpyDeviceToHost));
-            OWL_HIP(hipMemcpy(gC.data(), b->d_gC.get(), gC.size() * sizeof(double), hipMemcpyDeviceToHost));
-            std::vector<double> sv(nfull, 0.0), ss(nfull, 0.0), sr(nfull, 0.0);
-            for (size_t s = 0; s < b->sd.size(); ++s) {
-                const ShotHostE2& H = b->hs[s];
-                std::vector<double> gv, gs, gr;
-                window_grads_fs(b, s, gA.data(), gB.data(), gC.data(), gv, gs, gr);
-                for (int i = 1; i <= H.nx; ++i)
-                    for (int k = 1; k <= H.nz; ++k) {
-                        const size_t m = model_index2(b, H, i, k), o = size_t(k - 1) + size_t(i - 1) * H.nz;
-                        sv[m] += gv[o];
-                        ss[m] += gs[o];
-                        sr[m] += gr[o];
-                    }
-            }
-            for (size_t e = 0; e < nfull; ++e) {
-                if (grad_vp) grad_vp[e] = std::isfinite(sv[e]) ? sv[e] : 0.0;
-                if (grad_vs) grad_vs[e] = std::isfinite(ss[e]) ? ss[e] : 0.0;
-                if (grad_rho) grad_rho[e] = std::isfinite(sr[e]) ? sr[e] : 0.0;
-            }
-        } else if (grad_vp || grad_vs || grad_rho) {
+        if (grad_vp || grad_vs || grad_rho) {
             std::vector<double> fA(nfull), fB(nfull), fC(nfull);
             OWL_HIP(hipMemcpy(fA.data(), b->d_fA.get(), nfull * sizeof(double), hipMemcpyDeviceToHost));
             OWL_HIP(hipMemcpy(fB.data(), b->d_fB.get(), nfull * sizeof(double), hipMemcpyDeviceToHost));
             OWL_HIP(hipMemcpy(fC.data(), b->d_fC.get(), nfull * sizeof(double), hipMemcpyDeviceToHost));
             for (size_t e = 0; e < nfull; ++e) {
-                double gv, gs, gr;
-                chain_rule2(b->vp_full[e], b->vs_full[e], b->rho_full[e], fA[e], fB[e], fC[e], gv, gs, gr);
+                double gv = fA[e], gs = fB[e], gr = fC[e];  // of the free surface already through the chain rule
+                if (!b->fs) chain_rule2(b->vp_full[e], b->vs_full[e], b->rho_full[e], fA[e], fB[e], fC[e], gv, gs, gr);
                 if (grad_vp) grad_vp[e] = std::isfinite(gv) ? gv : 0.0;
                 if (grad_vs) grad_vs[e] = std::isfinite(gs) ? gs : 0.0;
                 if (grad_rho) grad_rho[e] = std::isfinite(gr) ? gr : 0.0;

@@ -368,27 +368,13 @@ void locate_ssg(const SsgMesh& m, float z, float oz, int& gz, int& hz, float* iz
     kaiser_sinc((z - oz - m.zh[size_t(hz + pml)]) / m.dzh[size_t(hz + pml)], hzw);
 }
 
-void column_to_regular_ssg(const SsgMesh& m, int nz0, const double* g, double* out) {
-    spline_to_regular(m.zi.data() + m.pml + 1, g, m.nz, m.dz, nz0, out);
-}
-
-void spline_to_regular(const float* x, const double* g, int n, float dz, int nz0, double* out) {
-    if (n < 3) fail(OWL_ERR_ARG, "too few refined rows");
-    std::vector<double> M(size_t(n), 0.0), cp(size_t(n), 0.0), dp(size_t(n), 0.0);
+void spline_table(const float* x, int n, std::vector<double>& out) {
+    const size_t cp = out.size(), den = cp + size_t(n);
+    out.resize(cp + 2 * size_t(n), 0.0);
     for (int i = 1; i < n - 1; ++i) {
         const double h0 = double(x[i]) - x[i - 1], h1 = double(x[i + 1]) - x[i];
-        const double r = 6.0 * ((g[i + 1] - g[i]) / h1 - (g[i] - g[i - 1]) / h0);
-        const double den = 2.0 * (h0 + h1) - h0 * cp[size_t(i - 1)];
-        cp[size_t(i)] = h1 / den;
-        dp[size_t(i)] = (r - h0 * dp[size_t(i - 1)]) / den;
-    }
-    for (int i = n - 2; i >= 1; --i) M[size_t(i)] = dp[size_t(i)] - cp[size_t(i)] * M[size_t(i + 1)];
-    for (int k = 0; k < nz0; ++k) {
-        const float v = float(k) * dz;
-        const int s = segment(x, n, v);
-        const double h = double(x[s + 1]) - x[s];
-        const double A = (double(x[s + 1]) - v) / h, B = (double(v) - x[s]) / h;
-        out[k] = A * g[s] + B * g[s + 1] + ((A * A * A - A) * M[size_t(s)] + (B * B * B - B) * M[size_t(s + 1)]) * h * h / 6.0;
+        out[den + size_t(i)] = 2.0 * (h0 + h1) - h0 * out[cp + size_t(i - 1)];
+        out[cp + size_t(i)] = h1 / out[den + size_t(i)];
     }
 }
 

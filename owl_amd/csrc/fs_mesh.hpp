@@ -104,14 +104,10 @@ void map_column_ssg(const SsgMesh& m, int nx, int nz0, const float* v, int i, fl
 // Kaiser-sinc of the offsets over dz_i(gz), dz_h(hz).
 void locate_ssg(const SsgMesh& m, float z, float oz, int& gz, int& hz, float* iz, float* hzw);
 
-// One window column of refined-row values g[j - 1], j = 1 .. nz, to the
-// regular rows 1 .. nz0 at (j - 1) dz by the natural cubic spline through
-// z_i(1 .. nz) (map_irregular_to_regular, module_vars.f90:175-203).
-void column_to_regular_ssg(const SsgMesh& m, int nz0, const double* g, double* out);
-
-// The natural cubic spline through (x[k], g[k]), k < n, at (k - 1) dz for
-// k = 1 .. nz0.
-void spline_to_regular(const float* x, const double* g, int n, float dz, int nz0, double* out);
+// The part of the natural cubic spline's tridiagonal elimination through
+// x[0 .. n-1] that does not depend on the values: appends cp and the
+// denominators, n each (Thomas sweep; rows 0 and n-1 zero).
+void spline_table(const float* x, int n, std::vector<double>& out);
 
 // Stable dt of the refined mesh (module_vars.f90:532-567): min over the
 // mesh of 1 / (sum|c| vmax dz0) with OWL's metric-scaled spacing.
