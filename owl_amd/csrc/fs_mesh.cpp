@@ -263,24 +263,6 @@ ZLoc locate_z(const Mesh& m, const Surface& s, float x, float z, bool source) {
     return L;
 }
 
-void to_regular(const Mesh& m, const float* g, float* out) {
-    const int nx = m.nx, nz = m.nz, nz0 = m.nz0;
-    std::vector<float> x(static_cast<size_t>(nz)), y(static_cast<size_t>(nz)), xq(static_cast<size_t>(nz0)), yq(static_cast<size_t>(nz0));
-    for (int j = 1; j <= nz0; ++j) xq[size_t(j - 1)] = float(j - 1) * m.dz0 - m.topo_max;
-    for (int i = 1; i <= nx; ++i) {
-        for (int j = 1; j <= nz; ++j) {
-            x[size_t(j - 1)] = m.zz_at(i, j);
-            y[size_t(j - 1)] = g[size_t(i - 1) + size_t(j - 1) * size_t(nx)];
-        }
-        ginterp(x.data(), y.data(), nz, xq.data(), nz0, yq.data(), true);
-        for (int j = 1; j <= nz0; ++j) {
-            const float zz = float(j - 1) * m.dz0;
-            out[size_t(j - 1) + size_t(i - 1) * size_t(nz0)] =
-                zz < m.topo_max - m.topo_i[size_t(i + m.pml)] ? 0.0f : yq[size_t(j - 1)];
-        }
-    }
-}
-
 SsgMesh build_ssg(int nx, int nz0, float dz, int pml, float refine, float dz_max, const float* c55, const float* rho,
                   float f0min) {
     if (nx < 1 || nz0 < 3) fail(OWL_ERR_ARG, "the free surface needs at least 3 rows");

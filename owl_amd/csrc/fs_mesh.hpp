@@ -1,10 +1,9 @@
 // OWL's free-surface mesh for the 2D FSG solver: the depth-refined,
 // topography-following mesh of one shot window (elastic_tti_2d/
 // module_vars.f90:360-519), the window's medium on it
-// (map_regular_to_irregular, :169-203), source and receiver rows on it
+// (map_regular_to_irregular, :169-203), and source and receiver rows on it
 // (:639-680 and the depth-varying branch of prepare_geometry,
-// src/lib/module_source_receiver.f90:556-760), and the refined-mesh
-// gradient back on the window (map_irregular_to_regular, :208-249).
+// src/lib/module_source_receiver.f90:556-760).
 //
 // OWL builds this with FLIT's regspace, deriv, rescale, ginterp and
 // pad_array, which are not part of the OWL tree.  They are taken as:
@@ -69,11 +68,6 @@ struct ZLoc {
     float amp_scale = 1.0f;
 };
 ZLoc locate_z(const Mesh& m, const Surface& s, float x, float z, bool source);
-
-// One refined-mesh gradient column set (nx, nz refined; x fastest) to the
-// window (nz0, nx) z fastest: the column's cubic interpolant at the regular
-// depths, zero above the free surface.
-void to_regular(const Mesh& m, const float* g, float* out);
 
 // The depth-refined mesh of OWL's 2D standard-staggered solver with a free
 // surface (elastic_vhtiort_2d/module_vars.f90:310-371): rows dz/refine
