@@ -301,15 +301,16 @@ owl_status owl_acoustic2d_observe(owl_acoustic2d *b);
  * stencil grid-point updates it performed. */
 owl_status owl_acoustic2d_last_stats(const owl_acoustic2d *b, double *ms, double *updates);
 
-/* Forward-step kernel of the exact-adjoint paths (no OWL counterpart;
+/* Step kernel of the forward, reverse and exact-adjoint passes (no OWL counterpart;
  * results are bit-identical either way): mode 0 two sweeps (p, then v)
  * and the two-pass adjoint, 1 one fused z-marching kernel per forward step
- * and per adjoint step, 2 fused for batches of 4 shots or more
- * (default).  zrows: z rows per fused tile (default 16).  The fused kernel needs
+ * and per adjoint step, 2 fused for batches of 4 shots or more that are
+ * large enough for it to be the faster one (default).  zrows: z rows per
+ * fused tile (before this call by the batch's size).  The fused kernel needs
  * distinct input and output states and no free surface; elsewhere the two
  * sweeps run. */
 owl_status owl_acoustic2d_set_step_kernel(owl_acoustic2d *b, int mode, int zrows);
-/* z rows per tile of the fused adjoint step (default 8; no OWL counterpart,
+/* z rows per tile of the fused adjoint step (no OWL counterpart;
  * results are bit-identical for any value). */
 owl_status owl_acoustic2d_set_adjoint_rows(owl_acoustic2d *b, int zrows);
 /* Autotuner of the fused kernels (no OWL counterpart): on (default), the

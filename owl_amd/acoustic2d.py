@@ -144,9 +144,9 @@ class Acoustic2DBatch:
         check(lib().owl_acoustic2d_set_graphs(self._h, int(bool(on))))
 
     def set_step_kernel(self, mode="auto", zrows=16):
-        """Forward-step kernel of the exact-adjoint paths: "sweeps" (p then
-        v), "fused" (one z-marching kernel per step) or "auto" (fused for 4
-        shots or more).  Results are bit-identical.  Turns the z-row
+        """Step kernel of the forward, reverse and exact-adjoint passes: "sweeps"
+        (p then v), "fused" (one z-marching kernel per step) or "auto" (fused
+        for 4 shots or more of a large enough batch).  Results are bit-identical.  Turns the z-row
         autotuner off."""
         m = {"sweeps": 0, "fused": 1, "auto": 2}[mode]
         check(lib().owl_acoustic2d_set_step_kernel(self._h, m, int(zrows)))

@@ -1386,14 +1386,14 @@ struct owl_acoustic2d {
     // exact adjoint: second working set, adjoint state, FP64 accumulators
     DevBuf<float> fM2[4];
     DevBuf<float> fC[3], fM3[4];      // third working set (fused steps ping-pong)
-    // fused forward step: 0 two sweeps, 1 fused, 2 fused for batches of
-    // 4 shots or more; z rows per tile
-    int step_kernel = 2, fzc = 16, nftile = 0;
+    // fused forward step: 0 two sweeps, 1 fused, 2 by the batch (adj_fused);
+    // z rows per tile, 0: set by the plan
+    int step_kernel = 2, fzc = 0, nftile = 0;
     std::vector<int> ftile_shot;
     DevBuf<int> d_ftile_shot;
     // fused adjoint: z rows per tile and its tile list; the autotuner picks
     // fzc and azc on the first exact gradient unless the caller set them
-    int azc = 8, natile = 0;
+    int azc = 0, natile = 0;
     std::vector<int> atile_shot;
     DevBuf<int> d_atile_shot;
     bool autotune = true, tuned = false;
@@ -1516,8 +1516,14 @@ void sweep_tiling(owl_acoustic2d* b) {
 }
 
 // Column-strip tiles of the fused step: 64 - (2R - 1) output columns and
-// fzc rows each, one wavefront per tile.
+// fzc rows each, one wavefront per tile: short tiles where their number would
+// leave the chip idle, long ones that recompute less where it does not.  us of
+// a forward step at 4 / 8 / 16 rows (R = 4, 461 x 461 nodes): 4 shots 19 / 20 /
+// 27, 8 shots 29 / 27 / 31, 16 shots 48 / 45 / 44, and of an adjoint step: 4
+// shots 32 / 37 / 53, 8 shots 56 / 56 / 67, 16 shots 113 / 106 / 105.
 void fused_tiling(owl_acoustic2d* b) {
+    if (b->fzc == 0) b->fzc = b->pts_full < 2.6e6 ? 8 : 16;
+    if (b->azc == 0) b->azc = b->pts_full < 1.2e6 ? 4 : 8;
     const int W = 64 - (2 * b->R - 1);
     b->ftile_shot.clear();
     for (size_t s = 0; s < b->sd.size(); ++s) {
@@ -2236,16 +2242,23 @@ bool offsets32(const owl_acoustic2d* b) {
     return b->field_elems < (size_t(1) << 28) && b->model_elems < (size_t(1) << 28);
 }
 
-// The fused adjoint step (k_adj_fused) runs wherever the fused forward step
-// may: batches of 4 shots or more by default, no free surface.
+// Whether the fused steps may run: no free surface, and by default 4 shots or
+// more with enough nodes to hide a tile's serial rows, of which the fused step
+// recomputes 2R - 1.  us of a forward / adjoint step of 4 and more shots,
+// sweeps against the better row count of fused: R = 4, 0.41 M nodes 12 / 18
+// against 14 / 20, 0.85 M 20 / 39 against 19 / 30, 1.7 M 35 / 74 against 27 /
+// 54; R = 6, 0.41 M 13 / 20 against 18 / 25, 0.85 M 21 / 40 against 25 / 41,
+// 1.7 M 36 / 77 against 33 / 70; R = 8, 1.7 M 38 / 80 against 43 / 77, 3.4 M 68
+// / 150 against 72 / 153, 6.8 M 136 / 298 against 123 / 299; R = 2, 0.41 M 11 /
+// 17 against 9 / 14.
 bool adj_fused(const owl_acoustic2d* b) {
     if (b->step_kernel == 0 || b->cfg.free_surface || !offsets32(b)) return false;
-    return !(b->step_kernel == 2 && b->sd.size() < 4);
+    if (b->step_kernel == 1) return true;
+    return b->sd.size() >= 4 && b->pts_full >= (b->R <= 4 ? 0.6e6 : b->R <= 6 ? 1.2e6 : 4.0e6);
 }
 
 bool use_fused(const owl_acoustic2d* b, const W7& in, const W7& out) {
-    if (b->step_kernel == 0 || b->cfg.free_surface || !offsets32(b)) return false;
-    if (b->step_kernel == 2 && b->sd.size() < 4) return false;
+    if (!adj_fused(b)) return false;
     for (int k = 0; k < 7; ++k)
         for (int m = 0; m < 7; ++m)
             if (in.f[k] == out.f[m]) return false;
