@@ -156,19 +156,57 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_p(const Shot* __restrict__
 // vx(m) = vx(m) - dt/(0.5*(rho(m)+rho(m-1))) * dx- p, PML where m <= 1 or
 // m >= nx+1; vz likewise along z.  One thread updates vx and vz at (i, j).
 // ---------------------------------------------------------------------------
-template <int R>
+// One receiver tap, as the sampling reads it: the element within the shot's
+// grid and two weights.  Shots whose receivers lie alike in like windows (a
+// fixed spread) share one table, which then stays in L2: 32 shots of 391
+// off-node receivers read 0.5 MB of taps per step instead of 16 MB.
+struct RecTap {
+    long long cell;
+    float w1, w2;
+};
+// The receivers of one step: `group` of a shot's per block, nrb blocks a shot
+// (nrb = 0: none).
+struct Sampling {
+    const int* beg;
+    const RecTap* taps;
+    const float* w;
+    float* traces;
+    int t, nrb, group;
+};
+__device__ __forceinline__ void sample_block(const Shot& S, int rb, const float* __restrict__ p, const Sampling& rec) {
+    const int r0 = rb * rec.group, r1 = min(r0 + rec.group, S.nr);
+    const float* ps = p + S.off;
+    ordered_sums(
+        r0, r1, [&](int r) { return rec.beg[S.rt0 + r]; },
+        [&](int k) {
+            const RecTap tp = rec.taps[k];
+            return ps[tp.cell] * tp.w1 * tp.w2;
+        },
+        [](int) { return 0.0f; }, [&](int r) { return rec.w[S.rec0 + r]; },
+        [&](int r, float acc) { rec.traces[S.trace0 + size_t(rec.t) * S.nr + r] = acc; });
+}
+
+// REC: the launch's first nrec blocks sample p, which this sweep only reads,
+// for the receivers.  A launch of their own, as bound by latency as the sweep
+// is, takes 4.2 us (one shot, 461 x 461 nodes, 391 receivers off the nodes);
+// here they add 1.0 us.
+template <int R, bool REC>
 __global__ __launch_bounds__(kBX * kBY) void k_update_v(const Shot* __restrict__ shots,
                                                         const int* __restrict__ tile_shot, Sets sets,
                                                         const float* __restrict__ rho,
                                                         const float* __restrict__ prof, Coef c,
                                                         float dt, float idx, float idz, int pml,
-                                                        int free_surface, int rpt) {
-    const int tile = blockIdx.x;
-    const Shot S = shots[shot_of_tile(tile_shot, tile)];
+                                                        int free_surface, int rpt, Sampling rec, int nrec) {
     const FieldSet F = sets.s[blockIdx.y];
+    if (REC && int(blockIdx.x) < nrec) {
+        sample_block(shots[blockIdx.x / rec.nrb], int(blockIdx.x) % rec.nrb, F.p_out, rec);
+        return;
+    }
+    const int tile = int(blockIdx.x) - (REC ? nrec : 0);
+    const Shot S = shots[shot_of_tile(tile_shot, tile)];
     const int lt = tile - S.tile0;
     const int tx = lt % S.ntx, tz = lt / S.ntx;
-    const int i = -pml + 1 + tx * kBX + int(threadIdx.x);
+    const int i = -pml + 1 + tx * kBX + int(threadIdx.x) % kBX;
     const int nx = S.nx, nz = S.nz;
     if (i > nx + pml) return;
     const int lo = 1 - pml - R;
@@ -187,7 +225,7 @@ __global__ __launch_bounds__(kBX * kBY) void k_update_v(const Shot* __restrict__
     const size_t pitch = size_t(S.pitch);
     for (int k = 0; k < rpt; ++k) {
         // kBX = 64: the row is wavefront-uniform (scalar registers)
-        const int j = -pml + 1 + tz * (kBY * rpt) + __builtin_amdgcn_readfirstlane(int(threadIdx.y)) + kBY * k;
+        const int j = -pml + 1 + tz * (kBY * rpt) + __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kBX) + kBY * k;
         if (j > nz + pml) break;
         const size_t q = size_t(S.off) + size_t(i - lo) + size_t(j - lo) * pitch;
         if (!free_surface || j >= 1) {
@@ -449,14 +487,6 @@ __global__ __launch_bounds__(256) void k_inject(const Shot* __restrict__ shots, 
     }
 }
 
-// One receiver tap, as the sampling reads it: the element within the shot's
-// grid and two weights.  Shots whose receivers lie alike in like windows (a
-// fixed spread) share one table, which then stays in L2: 32 shots of 391
-// off-node receivers read 0.5 MB of taps per step instead of 16 MB.
-struct RecTap {
-    long long cell;
-    float w1, w2;
-};
 // One adjoint-source tap (weights as in the sampling, then the receiver's).
 struct AdjTap {
     float w1, w2, rw;
@@ -470,27 +500,17 @@ constexpr int kStripsPerBlock = 1024;  // boundary-record elements a block copie
 template <int R>
 __global__ __launch_bounds__(kOrderedThreads) void k_record(
     const Shot* __restrict__ shots, const float* __restrict__ p, const float* __restrict__ vx,
-    const float* __restrict__ vz, int t, const int* __restrict__ rec_beg, const RecTap* __restrict__ rec_taps,
-    const float* __restrict__ rec_w, float* traces, float* strips, int nrb, int group, int pml) {
+    const float* __restrict__ vz, Sampling rec, float* strips, int pml) {
     const Shot S = shots[blockIdx.y];
-    if (int(blockIdx.x) < nrb) {
-        const int r0 = int(blockIdx.x) * group, r1 = min(r0 + group, S.nr);
-        const float* ps = p + S.off;
-        ordered_sums(
-            r0, r1, [&](int r) { return rec_beg[S.rt0 + r]; },
-            [&](int k) {
-                const RecTap tp = rec_taps[k];
-                return ps[tp.cell] * tp.w1 * tp.w2;
-            },
-            [](int) { return 0.0f; }, [&](int r) { return rec_w[S.rec0 + r]; },
-            [&](int r, float acc) { traces[S.trace0 + size_t(t) * S.nr + r] = acc; });
+    if (int(blockIdx.x) < rec.nrb) {
+        sample_block(S, int(blockIdx.x), p, rec);
         return;
     }
     const int nx = S.nx, nz = S.nz, lo = 1 - pml - R;
     const int na = R * (nz + 2 * R), nc = (nx + 2 * R) * R;
     const int len = 2 * na + 2 * nc;
-    float* rec = strips + S.strip0 + size_t(t) * len;
-    const int kb = (int(blockIdx.x) - nrb) * kStripsPerBlock;
+    float* strip = strips + S.strip0 + size_t(rec.t) * len;
+    const int kb = (int(blockIdx.x) - rec.nrb) * kStripsPerBlock;
     for (int k = kb + int(threadIdx.x); k < min(kb + kStripsPerBlock, len); k += blockDim.x) {
         int i, j;
         const float* src;
@@ -498,7 +518,7 @@ __global__ __launch_bounds__(kOrderedThreads) void k_record(
         else if (k < 2 * na) { const int kk = k - na; i = nx + 1 + kk % R; j = 1 - R + kk / R; src = vx; }
         else if (k < 2 * na + nc) { const int kk = k - 2 * na; i = 1 - R + kk % (nx + 2 * R); j = 2 - R + kk / (nx + 2 * R); src = vz; }
         else { const int kk = k - 2 * na - nc; i = 1 - R + kk % (nx + 2 * R); j = nz + 1 + kk / (nx + 2 * R); src = vz; }
-        rec[k] = src[size_t(S.off) + size_t(i - lo) + size_t(j - lo) * size_t(S.pitch)];
+        strip[k] = src[size_t(S.off) + size_t(i - lo) + size_t(j - lo) * size_t(S.pitch)];
     }
 }
 
@@ -1964,8 +1984,14 @@ StepBytes step_bytes(const owl_acoustic2d* b, int nsets) {
     return StepBytes{(bp + 4.0 * b->pts_model) * nsets, (bv + 4.0 * b->pts_model) * nsets};
 }
 
+Sampling sampling(const owl_acoustic2d* b, float* traces, int t) {
+    return Sampling{b->d_rec_beg.get(), b->d_rec_taps.get(), b->d_rec_w.get(), traces, t,
+                    (b->max_nr + b->rec_group - 1) / b->rec_group, b->rec_group};
+}
+
+// traces: null, or step t's receivers are sampled beside the v-sweep.
 template <int R>
-void launch_step(owl_acoustic2d* b, const Sets& sets, int nsets, float dt) {
+void launch_step(owl_acoustic2d* b, const Sets& sets, int nsets, float dt, float* traces = nullptr, int t = 0) {
     const int fs = b->cfg.free_surface ? 1 : 0;
     const dim3 blk(kBX, kBY), grd(unsigned(b->tile_shot.size()), unsigned(nsets));
     const StepBytes sb = b->profiling ? step_bytes(b, nsets) : StepBytes{0, 0};
@@ -1974,10 +2000,17 @@ void launch_step(owl_acoustic2d* b, const Sets& sets, int nsets, float dt) {
                        b->d_bk.get(), b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs, b->rpt);
     prof_end(b, ev);
     ev = prof_begin(b, nsets == 2 ? kKV2 : kKV, sb.v);
-    hipLaunchKernelGGL(k_update_v<R>, grd, blk, 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), sets,
-                       b->d_rho.get(), b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs, b->rpt);
+    const Sampling rec = sampling(b, traces, t);
+    const unsigned nrec = traces ? unsigned(rec.nrb) * unsigned(b->sd.size()) : 0;
+    hipLaunchKernelGGL(nrec ? (k_update_v<R, true>) : (k_update_v<R, false>), dim3(grd.x + nrec, grd.y),
+                       dim3(kBX * kBY), 0, b->stream, b->d_shots.get(), b->d_tile_shot.get(), sets, b->d_rho.get(),
+                       b->d_prof.get(), b->coef, dt, b->idx, b->idz, b->pml, fs, b->rpt, rec, int(nrec));
     prof_end(b, ev);
 }
+
+// Whether the receivers of step t+1 may be sampled beside step t's v-sweep: no
+// source adds to p after it.
+bool samples_with_v(const owl_acoustic2d* b, int t) { return t + 1 <= b->nt && (t < b->src_t0 || t > b->src_t1); }
 
 double fused_bytes(const owl_acoustic2d* b);
 bool adj_fused(const owl_acoustic2d* b);
@@ -2005,12 +2038,11 @@ void post_step(owl_acoustic2d* b, float* const* f, int t, float* traces, float* 
         prof_end(b, ev);
     }
     if (!traces || t + 1 > b->nt) return;
-    const int nrb = (b->max_nr + b->rec_group - 1) / b->rec_group;
+    const Sampling rec = sampling(b, traces, t);
     const int nsb = strips ? (b->max_strip + kStripsPerBlock - 1) / kStripsPerBlock : 0;
     const int ev = prof_begin(b, kKPost);
-    hipLaunchKernelGGL(k_record<R>, dim3(unsigned(nrb + nsb), nshot), dim3(kOrderedThreads), 0, b->stream,
-                       b->d_shots.get(), f[0], f[1], f[2], t, b->d_rec_beg.get(), b->d_rec_taps.get(),
-                       b->d_rec_w.get(), traces, strips, nrb, b->rec_group, b->pml);
+    hipLaunchKernelGGL(k_record<R>, dim3(unsigned(rec.nrb + nsb), nshot), dim3(kOrderedThreads), 0, b->stream,
+                       b->d_shots.get(), f[0], f[1], f[2], rec, strips, b->pml);
     prof_end(b, ev);
 }
 
@@ -2095,10 +2127,11 @@ void run_forward(owl_acoustic2d* b, bool save) {
         const SetPtr &in = cur ? C : A, &out = cur ? A : C;
         Sets sets{};
         sets.s[0] = sets.s[1] = field_set(in, out, out);
+        const bool beside = !fused && !save && samples_with_v(b, t);
         if (fused) launch_fused<R>(b, sets, 1, b->dt);
-        else launch_step<R>(b, sets, 1, b->dt);
+        else launch_step<R>(b, sets, 1, b->dt, beside ? b->d_traces.get() : nullptr, t);
         cur = 1 - cur;
-        post_step<R>(b, out.f, t, b->d_traces.get(), save ? b->d_strips.get() : nullptr);
+        post_step<R>(b, out.f, t, beside ? nullptr : b->d_traces.get(), save ? b->d_strips.get() : nullptr);
     }
     OWL_HIP(hipGetLastError());
     OWL_HIP(hipEventRecord(b->ev1, st));
@@ -2284,9 +2317,11 @@ void fwd_step(owl_acoustic2d* b, const W7& in, const W7& out, int t, bool record
         F.m_out[k] = out.f[3 + k];
     }
     sets.s[1] = F;
-    if (use_fused(b, in, out)) launch_fused<R>(b, sets, 1, b->dt);
-    else launch_step<R>(b, sets, 1, b->dt);
-    post_step<R>(b, out.f, t, record ? b->d_traces.get() : nullptr, nullptr);
+    float* traces = record ? b->d_traces.get() : nullptr;
+    const bool fused = use_fused(b, in, out), beside = traces && !fused && samples_with_v(b, t);
+    if (fused) launch_fused<R>(b, sets, 1, b->dt);
+    else launch_step<R>(b, sets, 1, b->dt, beside ? traces : nullptr, t);
+    post_step<R>(b, out.f, t, beside ? nullptr : traces, nullptr);
 }
 
 // Clear device memory on the batch stream: a memset, or a fill kernel while
