@@ -18,18 +18,17 @@ __device__ __forceinline__ int xcd_block() {
 
 // Rows (2D) or planes (3D) that one wavefront marches over, from the number
 // of wavefronts the batch has at one row or plane each.  A wavefront's march
-// is serial, a few us a row when few wavefronts share a SIMD, so a small
+// is serial, about 1.5 us a row when few wavefronts share a SIMD, so a small
 // batch wants as many wavefronts as it can have; a large one wants longer
 // marches, whose fill of the z queue (2R rows) weighs less.  The line is
 // where the chip holds about twice the wavefronts that run at once.
 // us per step on one MI355X at 2 / 4 / 8 / 32 rows: 2D elastic 301 x 201,
-// 1 shot 19 / 27 / 43 / 136, 8 shots 34 / 41 / 58 / 161, 32 shots 92 / 86 /
-// 84 / 188; FSG 333 x 171, 8 shots 58 / 59 / 81 / 227; 801 x 401, 32 shots
-// 723 / 688 / 687 / 783; 3D elastic 50 x 45 x 40 79 / 78 / 109 / 300, 117 x
-// 90 x 75, 2 shots 342 / 343 / 361 / 497; 200 x 200 x 150, 4 shots 3054 /
-// 2905 / 2891 / 3090; 3D acoustic (four-wide columns) 50 x 45 x 40 24 / 27 /
-// 39 / 106, 121 x 110 x 93, 2 shots 105 / 102 / 110 / 149, 256^3, 16 shots
-// 4499 / 4264 / 4203 / 4458.
+// 1 shot 14 / 17 / 22 / 59, 8 shots 25 / 27 / 33 / 69, 32 shots 59 / 60 / 67 /
+// 82; FSG 333 x 171, 8 shots 39 / 39 / 47 / 100; 801 x 401, 32 shots 514 / 477 /
+// 478 / 548; 3D elastic 50 x 45 x 40 61 / 57 / 70 / 175, 117 x 90 x 75, 2 shots
+// 259 / 248 / 263 / 313; 200 x 200 x 150, 4 shots 2430 / 2264 / 2243 / 2358; 3D
+// acoustic (four-wide columns) 50 x 45 x 40 24 / 27 / 39 / 106, 121 x 110 x 93,
+// 2 shots 105 / 102 / 110 / 149, 256^3, 16 shots 4499 / 4264 / 4203 / 4458.
 inline int default_planes(double wavefronts) {
     constexpr double kEnough = 14000.0;
     if (wavefronts / 8 >= kEnough) return 8;
