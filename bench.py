@@ -41,27 +41,21 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, GB/s
 # a timed process, so the values are carried here; profiles/ holds the
 # commands and the raw counts.
 TRAFFIC = {
-    # the fused 2D kernels at the z rows per tile the autotuner picks on this
-    # workload (acoustic2d_fwi_gradient_32shots.md)
-    ("acoustic2d_gradient", "step_fused", 16): (2.0 * 144.3e3 + 116.1e3) * 1024,
-    ("acoustic2d_gradient", "adjoint_fused", 8): (2.0 * 405.5e3 + 304.9e3) * 1024,
-    ("acoustic2d_gradient", "step_fused", 12): (2.0 * 151.9e3 + 115.1e3) * 1024,
-    ("acoustic2d_gradient", "adjoint_fused", 6): (2.0 * 433.9e3 + 306.3e3) * 1024,
-    ("acoustic3d_forward", "update_v"): (2.0 * 4.159e6 + 4.199e6) * 1024,    # acoustic3d_forward_256cube_16shots.md
-    ("acoustic3d_forward", "update_p"): (2.0 * 4.318e6 + 1.765e6) * 1024,
+    # the fused 2D kernels at these z rows per tile (acoustic2d_fwi_gradient_32shots.md)
+    ("acoustic2d_gradient", "step_fused", 16): (2.0 * 128.9e3 + 115.7e3) * 1024,
+    ("acoustic2d_gradient", "adjoint_fused", 8): (2.0 * 355.5e3 + 301.6e3) * 1024,
+    # (z planes, variant): acoustic3d_forward_256cube_16shots.md
+    ("acoustic3d_forward", "update_v", (8, 24)): (2.0 * 3.851e6 + 3.685e6) * 1024,
+    ("acoustic3d_forward", "update_p", (8, 24)): (2.0 * 3.643e6 + 1.586e6) * 1024,
     # (z planes, y rows per tile): elastic3d_forward_200x200x150_8shots.md
-    ("elastic3d_forward", "stress", (64, 4)): (2.0 * 6.017e6 + 2.686e6) * 1024,
-    ("elastic3d_forward", "velocity", (64, 4)): (2.0 * 5.066e6 + 1.602e6) * 1024,
-    ("elastic3d_forward", "stress", (8, 4)): (2.0 * 3.730e6 + 2.581e6) * 1024,
-    ("elastic3d_forward", "velocity", (8, 4)): (2.0 * 2.977e6 + 1.501e6) * 1024,
+    ("elastic3d_forward", "stress", (8, 4)): (2.0 * 3.569e6 + 2.682e6) * 1024,
+    ("elastic3d_forward", "velocity", (8, 4)): (2.0 * 2.845e6 + 1.486e6) * 1024,
     # (rows per tile column, tiles per block) of the FSG sweeps:
     # fsg2d_forward_free_surface_801x401_64shots.md
-    ("fsg2d_forward", "stress", (32, 4)): (2.0 * 7.750e5 + 3.767e5) * 1024,
-    ("fsg2d_forward", "velocity", (32, 4)): (2.0 * 4.983e5 + 2.834e5) * 1024,
-    ("fsg2d_forward", "stress", (8, 2)): (2.0 * 9.090e5 + 3.793e5) * 1024,
-    ("fsg2d_forward", "velocity", (8, 2)): (2.0 * 6.567e5 + 2.862e5) * 1024,
-    ("fsg2d_forward", "stress", (4, 2)): (2.0 * 9.996e5 + 3.790e5) * 1024,
-    ("fsg2d_forward", "velocity", (4, 2)): (2.0 * 8.005e5 + 2.863e5) * 1024,
+    ("fsg2d_forward", "stress", (8, 2)): (2.0 * 7.881e5 + 3.951e5) * 1024,
+    ("fsg2d_forward", "velocity", (8, 2)): (2.0 * 5.228e5 + 2.866e5) * 1024,
+    ("fsg2d_forward", "stress", (4, 2)): (2.0 * 6.964e5 + 3.820e5) * 1024,
+    ("fsg2d_forward", "velocity", (4, 2)): (2.0 * 4.318e5 + 2.770e5) * 1024,
 }
 
 
@@ -284,7 +278,7 @@ def bench_3d(sync, steps=1500, shape=None):
                         "dt 0.9 ms, R 4, pml 20, one HIP-graph launch of the time loop",
             "grid_pt_updates_per_s": updates / wall, "seconds": wall, "device_ms": ms,
             "eager_seconds_with_events": wall_eager,
-            "launch_shape": {"planes": kc, "variant": var}, "roofline": with_traffic("acoustic3d_forward", roof),
+            "launch_shape": {"planes": kc, "variant": var}, "roofline": with_traffic("acoustic3d_forward", roof, (kc, var)),
             "kernels": kernel_table(stats, 1)}
 
 
@@ -420,7 +414,7 @@ def bench_fsg(sync, steps, gradient=True, shape=None):
                 "algorithm": "OWL's gradient: forward with boundary records in HBM (FP16, one scale per shot "
                              "and step), L2 adjoint source per component (observed traces zero), reverse "
                              "reconstruction and adjoint, FP64 imaging of c11..c55 and rho on the refined "
-                             "meshes, mapped to the regular windows and summed on the host",
+                             "meshes, mapped to the regular windows and summed there",
                 "records": "fp16",
                 "finite": bool(all(np.isfinite(v).all() for v in g.values()))}
     b.close()

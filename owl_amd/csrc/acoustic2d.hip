@@ -188,7 +188,7 @@ __device__ __forceinline__ void sample_block(const Shot& S, int rb, const float*
 
 // REC: the launch's first nrec blocks sample p, which this sweep only reads,
 // for the receivers.  A launch of their own, as bound by latency as the sweep
-// is, takes 4.2 us (one shot, 461 x 461 nodes, 391 receivers off the nodes);
+// is, takes 4.2 us (one shot, 481 x 481 nodes, 391 receivers off the nodes);
 // here they add 1.0 us.
 template <int R, bool REC>
 __global__ __launch_bounds__(kBX * kBY) void k_update_v(const Shot* __restrict__ shots,
@@ -1517,7 +1517,7 @@ void upload_model(owl_acoustic2d* b) {
 // rows one after another (the stores keep the next row's loads behind them),
 // so a small batch gives every row a thread of its own and a large one,
 // which fills the chip anyway, reads its block's tables once for 4 rows.  us
-// per forward step at 1 / 2 / 4 rows: 461 x 461 nodes, 1 shot 13.4 / 15.6 /
+// per forward step at 1 / 2 / 4 rows: 481 x 481 nodes, 1 shot 13.4 / 15.6 /
 // 20.4, 2 shots 16.2 / 17.9 / 22.7, 4 shots 23.0 / 21.8 / 26.0, 8 shots 35.9
 // / 33.5 / 32.2, 16 shots 57.0 / 53.5 / 51.9.
 void sweep_tiling(owl_acoustic2d* b) {
@@ -1538,7 +1538,7 @@ void sweep_tiling(owl_acoustic2d* b) {
 // Column-strip tiles of the fused step: 64 - (2R - 1) output columns and
 // fzc rows each, one wavefront per tile: short tiles where their number would
 // leave the chip idle, long ones that recompute less where it does not.  us of
-// a forward step at 4 / 8 / 16 rows (R = 4, 461 x 461 nodes): 4 shots 19 / 20 /
+// a forward step at 4 / 8 / 16 rows (R = 4, 481 x 481 nodes): 4 shots 19 / 20 /
 // 27, 8 shots 29 / 27 / 31, 16 shots 48 / 45 / 44, and of an adjoint step: 4
 // shots 32 / 37 / 53, 8 shots 56 / 56 / 67, 16 shots 113 / 106 / 105.
 void fused_tiling(owl_acoustic2d* b) {
@@ -2148,7 +2148,7 @@ void run_forward(owl_acoustic2d* b, bool save) {
 // OWL's reverse loop t = nt .. hnt (submodule_fwi_gradient.f90:75-167).
 // Where the fused step may run (adj_fused) both field sets advance by it, out
 // of place with their memory variables: one launch of 156 us for 32 shots of
-// 461 x 461 nodes in place of 254 us of sweeps.  (Running 10 or 16 of the
+// 481 x 481 nodes in place of 254 us of sweeps.  (Running 10 or 16 of the
 // shots at a time, so that a step finds its fields in the last-level cache,
 // gained nothing.)
 template <int R>
@@ -2279,10 +2279,10 @@ bool offsets32(const owl_acoustic2d* b) {
 // more with enough nodes to hide a tile's serial rows, of which the fused step
 // recomputes 2R - 1.  us of a forward / adjoint step of 4 and more shots,
 // sweeps against the better row count of fused: R = 4, 0.41 M nodes 12 / 18
-// against 14 / 20, 0.85 M 20 / 39 against 19 / 30, 1.7 M 35 / 74 against 27 /
-// 54; R = 6, 0.41 M 13 / 20 against 18 / 25, 0.85 M 21 / 40 against 25 / 41,
-// 1.7 M 36 / 77 against 33 / 70; R = 8, 1.7 M 38 / 80 against 43 / 77, 3.4 M 68
-// / 150 against 72 / 153, 6.8 M 136 / 298 against 123 / 299; R = 2, 0.41 M 11 /
+// against 14 / 20, 0.93 M 20 / 39 against 19 / 30, 1.85 M 35 / 74 against 27 /
+// 54; R = 6, 0.41 M 13 / 20 against 18 / 25, 0.93 M 21 / 40 against 25 / 41,
+// 1.85 M 36 / 77 against 33 / 70; R = 8, 1.85 M 38 / 80 against 43 / 77, 3.7 M 68
+// / 150 against 72 / 153, 7.4 M 136 / 298 against 123 / 299; R = 2, 0.41 M 11 /
 // 17 against 9 / 14.
 bool adj_fused(const owl_acoustic2d* b) {
     if (b->step_kernel == 0 || b->cfg.free_surface || !offsets32(b)) return false;
